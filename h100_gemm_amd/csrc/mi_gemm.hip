@@ -23,7 +23,7 @@
 
 namespace mi {
 hipError_t launch_reference_gpu_gemm(int dtype, int M, int N, int K, const void* A, const void* B,
-                                     void* C, float alpha, float beta, hipStream_t stream);
+                                     void* C, float alpha, float beta, int cus, hipStream_t stream);
 }
 
 namespace {
@@ -812,7 +812,7 @@ int mi_reference_gpu_gemm(int dtype, int M, int N, int K, const void* A, const v
     int rc = check_args(MI_CONFIG_AUTO, dtype, M, N, K, A, B, C);
     if (rc != MI_OK) return rc;
     hipError_t err =
-        mi::launch_reference_gpu_gemm(dtype, M, N, K, A, B, C, alpha, beta, (hipStream_t)stream);
+        mi::launch_reference_gpu_gemm(dtype, M, N, K, A, B, C, alpha, beta, compute_units(), (hipStream_t)stream);
     if (err != hipSuccess)
         return fail(MI_ERR_HIP, "launch of the reference GEMM failed: %s", hipGetErrorString(err));
     return MI_OK;

@@ -881,6 +881,34 @@ def test_reference_gpu_gemm_is_bit_identical_to_the_oracle(mi, orc):
         assert (dC.to_numpy((M, N), np.uint16) == orc.reference_cpu_gemm(A, B, alpha=0.5, beta=0.25)).all()
 
 
+# the tile widths the golden picks by the number of tiles: 4, 8, 16, 32 and 64 columns per wave; rows
+# and columns that end inside a tile, K below, at and just past whole 64-deep units (a ring shorter and
+# longer than its stages), every length of the last 16-byte piece
+@pytest.mark.parametrize("M,N,K", [(1, 1, 1), (65, 15, 63), (64, 16, 64), (63, 17, 65), (513, 509, 130), (129, 33, 327),
+                                   (513, 1023, 77), (1021, 1024, 196), (1023, 2047, 129), (2047, 2045, 71),
+                                   (2048, 2048, 320)])
+@pytest.mark.parametrize("dtype", [0, 1])
+def test_reference_gpu_gemm_every_tile_width_is_bit_identical(mi, orc, M, N, K, dtype):
+    """Exact, on the alpha / beta epilogue with C at an odd element offset too, and where products and
+    sums are subnormal in fp32: small integers times 2^-70, whose products are whole multiples of
+    2^-140 (a product that is itself rounded is another matter: the kernel's is an fma's)."""
+    print(f"case golden M={M} N={N} K={K} dtype={dtype}", flush=True)
+    tiny = dtype == 0 and K % 2 == 1
+    A, B = make_inputs(orc, M, N, K, "int" if tiny else "uniform", dtype)
+    if tiny:                                             # bf16 exponents lowered by 70, zeros left alone
+        A, B = [np.where((x & 0x7FFF) != 0, x - (70 << 7), x).astype(np.uint16) for x in (A, B)]
+    dA, dB = mi.DeviceBuffer.from_numpy(A), mi.DeviceBuffer.from_numpy(B)
+    dC = mi.DeviceBuffer(M * N * 2 + 16)
+    for alpha, beta, off in [(1.0, 0.0, 0), (0.5, 0.25, 2)]:
+        dC.fill_bytes(0xFF)
+        mi.reference_gpu_gemm(mi.GemmParams(M, N, K, dA, dB, dC.ptr + off, alpha, beta), dtype=dtype)
+        mi.synchronize()
+        got = dC.to_numpy((M * N + 8,), np.uint16)
+        ref = orc.reference_cpu_gemm(A, B, dtype=dtype, alpha=alpha, beta=beta)
+        assert (got[off // 2:off // 2 + M * N].reshape(M, N) == ref).all()
+        assert (got[:off // 2] == 0xFFFF).all() and (got[off // 2 + M * N:] == 0xFFFF).all()
+
+
 # ------------------------------------------------------------------ trace buffer ------
 
 def test_db_trace_records(mi, orc):
