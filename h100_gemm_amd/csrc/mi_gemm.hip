@@ -18,6 +18,7 @@
 
 #include "../../include/mi_gemm.h"
 #include "gemm_kernel.hpp"
+#include "pack_kernel.hpp"
 #include "splitk_common.hpp"   // splitk_reduce_kernel
 #include "kernel_table.hpp"
 
@@ -173,6 +174,9 @@ struct DeviceState {
 // grow the table beyond this: the next new stream waits for the device to go idle and takes over
 // an entry (see acquire_workspace), so at most this many live buffers exist per device.
 constexpr size_t kMaxStreamWs = 16;
+// Most a launch takes of it for a copy of its operands (choose_packing); larger ones run on the
+// operands as they are.
+constexpr size_t kMaxPackedBytes = (size_t)2 << 30;
 std::mutex g_ws_mutex;
 DeviceState g_dev[kMaxDevices];
 
@@ -208,7 +212,9 @@ void free_entry(StreamWs& w) {
 
 // 0: *out holds `bytes` of workspace; 1: none to be had without allocating where that is not
 // possible (the caller runs the launch unsplit); < 0: MI_ERR_* with the message set.
-int acquire_workspace(const WsSource& src, size_t bytes, hipStream_t stream, float** out) {
+// `required` false: the caller can do without, so no other stream's entry is taken over and a
+// failed allocation is 1.
+int acquire_workspace(const WsSource& src, size_t bytes, hipStream_t stream, float** out, bool required = true) {
     *out = nullptr;
     if (src.mode == WS_CALLER) {
         if (!src.ptr || src.bytes < bytes) return 1;
@@ -245,6 +251,7 @@ int acquire_workspace(const WsSource& src, size_t bytes, hipStream_t stream, flo
     size_t want = (size_t)4 << 20;
     while (want < bytes) want <<= 1;
     if (!mine && st.ws.size() >= kMaxStreamWs) {
+        if (!required) return 1;
         // The table is full (a process that keeps making streams, or never releases): once the
         // device is idle no launch holds any buffer, so the smallest entry changes hands -- its
         // buffer as it is when large enough, else freed here and replaced below.
@@ -270,7 +277,15 @@ int acquire_workspace(const WsSource& src, size_t bytes, hipStream_t stream, flo
         mine = take;
     }
     float* p = nullptr;
+    // (relaxed for this thread: the allocation concerns no capture another thread has under way)
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
     hipError_t e = hipMalloc((void**)&p, want);
+    if (relaxed) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (e != hipSuccess && !required) {
+        (void)hipGetLastError();
+        return 1;
+    }
     if (e != hipSuccess)
         return fail(MI_ERR_HIP, "split-K workspace allocation of %zu bytes failed: %s", want, hipGetErrorString(e));
     if (mine) {
@@ -282,6 +297,15 @@ int acquire_workspace(const WsSource& src, size_t bytes, hipStream_t stream, flo
     }
     *out = p;
     return 0;
+}
+
+bool is_capturing(hipStream_t stream) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &cap) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;       // e.g. the null stream while another stream captures
+    }
+    return cap != hipStreamCaptureStatusNone;
 }
 
 int compute_units() {
@@ -416,6 +440,49 @@ Choice choose(int requested, int M, int N, int K, bool streamable, bool splittab
     memo[next] = c;
     next = (next + 1) & 3;
     return c;
+}
+
+// Which operands of a tiled launch are first copied to rows that start on 128-byte lines
+// (pack_operands_kernel), a pure function of the choice and the shape.
+//
+// With K % 64 != 0 the K loop of the 16x16x32 kernel runs at 0.69-0.83 of its rate on whole lines
+// (4095 x 6143 with K = 3073 / 3072: 180.7 / 124.6 us; 8191^3 941, 8191 x 8191 x 8192 725).  What
+// the copy saves grows with M*N*K: per product of extents 9e-10 us with tiles whose loads bound
+// the step (256x192: 6.5-8.9e-10; 192x192: 8-10.7e-10; 128x256: 11e-10), 3.2e-10 with the 256x256
+// tile, whose MFMAs hide part of the loads (2.8-4.4e-10), and a copy of one operand alone saves half
+// of that or less.  It costs its launch and 7.5e-7 us per element copied (5 TB/s).  None / A / B / both in us:
+// 4095x6143x3073 181 / 167 / 168 / 145, 3000^3 67 / 74 / 72 / 63, 2100x2100x9000 in two pieces
+// 109 / 118 / 116 / 99, 2048x28672x4100 454 / 408 / 488 / 457, 28672x2048x4100 482 / 500 / 454 / 463,
+// 8192x8192x8200 858 / 816 / 842 / 817; not worth it: 2048x2048x2049 29 / 35 / 34 / 32,
+// 4000x4000x600 31 / 37 / 40 / 39.
+struct PackPlan {
+    bool a, b;
+    bool any() const { return a || b; }
+    size_t bytes(int M, int N, int K) const {
+        return ((a ? (size_t)M : 0) + (b ? (size_t)N : 0)) * (size_t)((K + 63) / 64 * 64) * 2;
+    }
+};
+PackPlan choose_packing(const Choice& c, int M, int N, int K) {
+    const mi::KernelEntry& e = mi::kKernels[c.config];
+    PackPlan best{false, false};
+    if (K % 64 == 0 || e.kind != mi::KIND_MFMA16 || e.kg > 1) return best;
+    const double mnk = (double)M * N * K;
+    const bool square = e.BM == 256 && e.BN == 256;
+    double best_gain = 3.6e-11 * mnk;                        // 2 % of the launch at 1.1 PFLOP/s
+    for (int which = 1; which <= 3; ++which) {
+        const PackPlan p{(which & 1) != 0, (which & 2) != 0};
+        if (p.bytes(M, N, K) > kMaxPackedBytes) continue;
+        const double saves = (which == 3 ? (square ? 3.2e-10 : 9.0e-10) : (square ? 1.6e-10 : 3.0e-10)) * mnk;
+        const double gain = saves - 4.0 - 7.5e-7 * ((p.a ? (double)M : 0.0) + (p.b ? (double)N : 0.0)) * K;
+        if (gain > best_gain) {
+            best = p;
+            best_gain = gain;
+        }
+    }
+    return best;
+}
+size_t choice_workspace(const Choice& c, int M, int N, int K) {
+    return choose_packing(c, M, N, K).bytes(M, N, K) + (c.splits > 1 ? (size_t)c.splits * M * N * sizeof(float) : 0);
 }
 
 // The cut of a large ragged shape into two GEMMs is a pure function of the shape and four flags
@@ -559,22 +626,53 @@ int run_gemm(int config, int dtype, int M, int N, int K, const void* A, const vo
     if (e.kg > 1 && K % (128 * e.kg) != 0)
         return fail(MI_ERR_UNSUPPORTED, "config %s splits K over %d groups of waves and needs K %% %d == 0", e.name,
                     e.kg, 128 * e.kg);
-    const bool edge = !shape_is_aligned(e, M, N, K, A, B, C);
-    mi::LaunchFn fn = e.launch[dtype][edge ? 1 : 0];
-    if (!fn) return fail(MI_ERR_UNSUPPORTED, "config %s has no %s kernel for dtype %d", e.name,
-                         edge ? "predicated" : "aligned", dtype);
     if (e.kind == mi::KIND_MFMA16) {
         args.splits = choice.splits;
         args.k_per_split = choice.k_per_split;
-        if (args.splits > 1) {
-            const int wrc = acquire_workspace(wsrc, (size_t)args.splits * M * N * sizeof(float), (hipStream_t)stream, &args.ws);
+        const size_t split_bytes = args.splits > 1 ? (size_t)args.splits * M * N * sizeof(float) : 0;
+        // The copy of the operands is an option: without room for it (the static array, a caller's
+        // workspace that is too small, no memory) the launch runs on the operands as they are, to the
+        // same bits.  Not from the library's buffer under capture: a graph of such a launch needed
+        // no workspace and may be replayed on any stream.
+        PackPlan plan = choose_packing(choice, M, N, K);
+        float* room = nullptr;
+        if (plan.any() && (wsrc.mode == WS_STATIC || (wsrc.mode == WS_CALLER && ((uintptr_t)wsrc.ptr & 127u) != 0) ||
+                           (wsrc.mode == WS_LIBRARY && is_capturing((hipStream_t)stream)) ||
+                           acquire_workspace(wsrc, plan.bytes(M, N, K) + split_bytes, (hipStream_t)stream, &room, false) != 0))
+            plan = {false, false};
+        if (plan.any()) {
+            unsigned char* packed = (unsigned char*)room;
+            const int pitch = (K + 63) / 64 * 64;
+            mi::PackArgs pa;
+            pa.src[0] = (const uint16_t*)(plan.a ? A : B);
+            pa.src[1] = (const uint16_t*)B;
+            pa.out = (uint16_t*)packed;
+            pa.rows_first = (uint32_t)(plan.a ? M : N);
+            pa.chunks = (uint32_t)pitch / 8u;
+            pa.total = (pa.rows_first + (plan.a && plan.b ? (uint32_t)N : 0u)) * pa.chunks;
+            pa.K = K;
+            const uint32_t per_block = 256u * mi::kPackChunks;
+            hipError_t err = mi::launch_kernel(mi::pack_operands_kernel, dim3((pa.total + per_block - 1) / per_block), dim3(256),
+                                               (hipStream_t)stream, pa);
+            if (err != hipSuccess) return fail(MI_ERR_HIP, "launch of the operand copy failed: %s", hipGetErrorString(err));
+            if (plan.a) { args.A = packed; args.lda = pitch; }
+            if (plan.b) { args.B = packed + (plan.a ? (size_t)M * pitch * 2 : 0); args.ldb = pitch; }
+            if (plan.a && plan.b) args.K = pitch;       // both end in zeros: no K tail
+            if (split_bytes) args.ws = (float*)(packed + plan.bytes(M, N, K));
+        } else if (args.splits > 1) {
+            const int wrc = acquire_workspace(wsrc, split_bytes, (hipStream_t)stream, &args.ws);
             if (wrc < 0) return wrc;
             if (wrc > 0) {
                 args.splits = 1;
                 args.k_per_split = K;
             }
         }
+        if (args.splits == 1) args.k_per_split = args.K;
     }
+    const bool edge = !shape_is_aligned(e, M, N, args.K, args.A, args.B, C);
+    mi::LaunchFn fn = e.launch[dtype][edge ? 1 : 0];
+    if (!fn) return fail(MI_ERR_UNSUPPORTED, "config %s has no %s kernel for dtype %d", e.name,
+                         edge ? "predicated" : "aligned", dtype);
     hipError_t err = fn(args, (hipStream_t)stream);
     if (err != hipSuccess)
         return fail(MI_ERR_HIP, "launch of %s failed: %s", e.name, hipGetErrorString(err));
@@ -735,7 +833,7 @@ size_t mi_gemm_workspace_bytes(int config, int dtype, int M, int N, int K, int c
                 // may split where one that can does not: both cases)
                 for (int small = 0; small < 2; ++small) {
                     const Choice c = compute_choice(config, rows, N, K, streamable != 0, N % 4 == 0, aligned != 0, small != 0);
-                    const size_t b = c.splits > 1 ? (size_t)c.splits * rows * N * sizeof(float) : 0;
+                    const size_t b = choice_workspace(c, rows, N, K);
                     if (b > need) need = b;
                 }
         return need;

@@ -74,7 +74,11 @@ int mi_gemm_epilogue(int config, int dtype, int M, int N, int K, const void* A, 
 /* ---- split-K workspace -----------------------------------------------------------------
  * Shapes with few output tiles and a long K (decode shapes with 32 < M <= 128, 128 x 384 x
  * 13376, 800 x 800 x 6000, ...) run as split-K: fp32 partial sums [pieces][M][N] go to a workspace and a second
- * kernel adds them in a fixed order.  The three entry points above take that workspace from
+ * kernel adds them in a fixed order.  Large shapes with K % 64 != 0 (4095 x 6143 x 3073) use the
+ * same workspace for a copy of A, B or both with rows on 128-byte lines, at most 2 GiB; the copy
+ * changes no bit of the result and is left out where there is no room for it: on a capturing
+ * stream, when the allocation fails, when 16 other streams hold buffers, with a caller's workspace
+ * that is too small, and always in mi_gemm_bf16_noalloc.  The three entry points above take that workspace from
  * the library: one buffer per (device, stream), a power of two of at least 4 MiB, allocated on
  * the first call that needs it and replaced by a larger one on demand; a replaced buffer is
  * kept (an enqueued launch or a captured graph may still hold its address) until
@@ -85,7 +89,7 @@ int mi_gemm_epilogue(int config, int dtype, int M, int N, int K, const void* A, 
  * be replayed afterwards, as after a release: captured work that shares a process with more
  * than 16 GEMM streams should bring its own workspace).  A stream under capture that has no large enough buffer yet runs the launch unsplit;
  * a first or a growing use calls hipMalloc, which must not happen while ANY thread captures
- * in hipStreamCaptureModeGlobal: reserve beforehand (mi_gemm_reserve_workspace) or use
+ * in hipStreamCaptureModeGlobal (the library asks for it in relaxed mode): reserve beforehand (mi_gemm_reserve_workspace) or use
  * mi_gemm_epilogue_ws / mi_gemm_bf16_noalloc there.  The reference's launchers allocate
  * nothing per call (matmul_h100_optimal.cu:32-59); mi_gemm_epilogue_ws gives a caller the
  * same property: it owns the workspace, per stream or per graph, and the library allocates
@@ -111,7 +115,7 @@ int mi_gemm_release_workspace(void* stream);
 size_t mi_gemm_library_workspace_bytes(void);
 
 /* Bytes of workspace the library's choice of kernel wants for this call (0 when the shape
- * does not run split-K).  An upper bound: the largest need over the pointer alignments a
+ * neither runs split-K nor copies its operands).  An upper bound: the largest need over the pointer alignments a
  * launch can meet and over the two parts of a shape whose rows the automatic choice cuts
  * (2248 x 8192 x 28672: 140.5 MiB for the uncut split of an unaligned call, 25 MiB for the
  * aligned call, which is cut at 2048 rows). */

@@ -686,6 +686,43 @@ def test_caller_workspace_launches_on_two_streams(mi, orc):
         assert hip.hipStreamDestroy(s) == 0
 
 
+# A and B are copied to whole-line rows first (both; A alone; B alone; with K in pieces), and not: K % 64
+# of 1, 63 and 8, rows and columns at the edges of the tiles
+@pytest.mark.parametrize("M,N,K,copied", [(2817, 2819, 2753, "AB"), (2500, 3000, 2623, "AB"), (2560, 3072, 2568, "AB"),
+                                          (2048, 28672, 1089, "A"), (28673, 2049, 1096, "B"), (2100, 2100, 9001, "AB"),
+                                          (1024, 1024, 1025, "")])
+def test_operands_copied_to_whole_lines_change_no_bit(mi, orc, M, N, K, copied):
+    """With a ragged K a large launch copies its operands to rows on 128-byte lines in its workspace.
+    The same kernel then adds the same products in the same order (zeros at the end of a row add
+    nothing): with room for the copy and without, C is the same bit for bit, and the tolerance
+    holds on sampled tiles.  The workspace starts as NaN: what is read of it was written."""
+    L = mi._lib.load()
+    for dtype in (0, 1):
+        A, B = make_inputs(orc, M, N, K, "normal", dtype)
+        d = Dev(mi, A, B, M, N)
+        need = mi.workspace_bytes(M, N, K, dtype=dtype)
+        pitch = (K + 63) // 64 * 64
+        rows = ("A" in copied) * M + ("B" in copied) * N
+        splits = need - rows * pitch * 2
+        assert splits >= 0 and splits % (M * N * 4) == 0, (need, rows)
+        ws = mi.DeviceBuffer(max(need, 16))
+        ws.fill_bytes(0xFF)
+        got = []
+        # (the last: room for the pieces' sums, not for the copy)
+        for ptr, size in [(ws.ptr, need), (ws.ptr, splits)]:
+            d.dC.fill_bytes(0xFF)
+            mi._lib.check(L.mi_gemm_epilogue_ws(-1, dtype, M, N, K, d.dA.ptr, d.dB.ptr, d.dC.ptr, 1.0, 0.0, 0, ptr, size, None))
+            mi.synchronize()
+            got.append(d.dC.to_numpy((M, N), np.uint16).copy())
+        assert (got[0] == got[1]).all(), f"dtype {dtype}: {int((got[0] != got[1]).sum())} elements differ"
+        assert (d.run(K, dtype=dtype) == got[0]).all()               # the library's own workspace
+        tiles = orc.sample_tiles(M, N, 16)
+        ref = orc.reference_cpu_gemm(A, B, dtype=dtype, tiles=tiles)
+        rep = orc.check_tolerance(got[0], ref, K, orc.max_abs(A, dtype), orc.max_abs(B, dtype), dtype, tiles=tiles)
+        assert rep["violations"] == 0 and rep["compared"] > 0, rep
+    mi._lib.check(L.mi_gemm_release_workspace(None))
+
+
 def test_hip_graph_replay_of_gemm_launches(mi, orc):
     """A launch is kernel launches only and can be captured into a HIP graph: a tiled, a decode
     and two split-K GEMMs (caller workspaces) recorded on a capturing stream, plus one split-K
