@@ -4,19 +4,24 @@
 //
 // B (the weights) is read exactly once from HBM and that read is the whole cost, so the
 // kernel is a set of independent streams, one per wave:
-//   * a workgroup owns 32 rows of B (32 columns of C) over all of K; N = 8192 gives one
-//     workgroup per CU;
+//   * a workgroup owns BN = 8, 16, 24 or 32 rows of B (columns of C) over all of K.  A CU takes in
+//     ~26 GB/s whatever it keeps in flight, so BN is the narrowest that keeps N / BN workgroups
+//     within one round of the CUs (stream_time_us in the kernel table): 1 x 4096 x 4096 with 32
+//     columns on 128 workgroups 9.2 us (3.6 TB/s), with 16 on 256 7.1 (4.7); 1 x 2048 x 4096 with 8
+//     5.2, 16 x 6144 x 4096 with 24 10.2 (32: 11.3).  Narrower still reads more of A, which every
+//     workgroup walks whole: 16 x 8192 x 8192 with 32 21.9 us, with 16 24.0, with 8 30.2;
 //   * its four waves split K between them, 64-deep slab by slab (wave w takes slabs
 //     w, w+4, ...), so the workgroup as a whole walks 512 contiguous bytes of every row;
 //   * each wave has a private ring of NS stages in LDS, filled by direct-to-LDS buffer
 //     loads (B rows and the matching k range of A, 128-byte rows, XOR-swizzled) and
-//     drained by its own MFMAs; a wave waits only on its own `vmcnt`, there is no barrier
-//     in the loop, and NS-1 slabs per wave are always in flight;
+//     drained by its own MFMAs (32x32x16 with 24 or 32 columns, 16x16x32 with fewer); a wave
+//     waits only on its own `vmcnt`, there is no barrier in the loop, and NS-1 slabs per wave
+//     are always in flight (narrow stages are small: rings of five where 32 columns have three);
 //   * workgroup b starts its walk over K at slab 37*b mod K/64 and wraps around: with every
 //     workgroup at the same k at the same time, all requests in flight would share their
 //     low address bits (rows are K*2 bytes apart) and crowd a few HBM channels; staggered
 //     starts measured 6.7 TB/s against 4.7 TB/s for the same bytes;
-//   * the four partial 32x32 fp32 tiles are added in wave order through LDS (a fixed order:
+//   * the four partial fp32 tiles are added in wave order through LDS (a fixed order:
 //     results are reproducible), rounded once and stored.
 // A is re-read by every workgroup; it is at most 64 x K and stays in L2.
 // Rows of A past M and rows of B past N are never fetched (the buffer descriptors end at
@@ -28,23 +33,28 @@
 #include <stdint.h>
 
 #include "gemm_kernel.hpp"
+#include "gemm_mfma16_kernel.hpp"   // mfma_16x16x32
 #include "splitk_common.hpp"
 
 namespace mi {
 
-template <int BM_, int NS_, int DT_>
+template <int BM_, int NS_, int DT_, int BN_ = 32>
 struct StreamConfig {
-    static constexpr int BM = BM_, BN = 32, NS = NS_, DT = DT_;
+    static constexpr int BM = BM_, BN = BN_, NS = NS_, DT = DT_;
     static constexpr int NT = 256, NW = 4;
     static constexpr int ROWS = BM + BN;                     // rows of one stage: A then B
     static constexpr int STAGE = ROWS * 128;
     static constexpr int L = ROWS / 8;                       // load instructions per slab
     static constexpr int RING = NS * STAGE;                  // one wave's ring
     static constexpr int LDS_BYTES = NW * RING;
-    static constexpr int MI = (BM + 31) / 32;                // 32-row MFMA blocks of A
-    static_assert(BM == 16 || BM % 32 == 0, "A block is half of or whole 32-row MFMA operands");
+    static constexpr bool WIDE = BN > 16;                   // 32x32x16 MFMAs, else 16x16x32
+    static constexpr int R = WIDE ? 32 : 16;                 // rows and columns of an MFMA block
+    static constexpr int KS = WIDE ? 4 : 2;                  // MFMAs deep a slab is
+    static constexpr int MI = (BM + R - 1) / R;              // MFMA blocks of A
+    static_assert(BN == 32 || BN == 24 || BN == 16 || BN == 8, "columns of a workgroup: one MFMA block or part of one");
+    static_assert(BM == 16 || BM % 32 == 0, "A block is half of or whole MFMA operands");
     static_assert(NS >= 2 && (NS - 1) * L <= 63, "vmcnt is a 6-bit counter");
-    static_assert(RING >= MI * 32 * 32 * 4, "a ring holds the wave's fp32 partial tile");
+    static_assert(RING >= MI * R * R * 4, "a ring holds the wave's fp32 partial tile");
     static_assert(LDS_BYTES <= 160 * 1024, "LDS budget of one CU");
 };
 
@@ -54,6 +64,8 @@ template <class Cfg, bool TRACE = false>
 __global__ void __launch_bounds__(256) gemm_stream_kernel(const DecodeArgs p) {
     constexpr int BM = Cfg::BM, NS = Cfg::NS, DT = Cfg::DT;
     constexpr int L = Cfg::L, STAGE = Cfg::STAGE, RING = Cfg::RING, MI = Cfg::MI;
+    constexpr int BN = Cfg::BN, R = Cfg::R, KS = Cfg::KS;
+    constexpr bool WIDE = Cfg::WIDE;
 
     __shared__ __attribute__((aligned(128))) unsigned char lds[Cfg::LDS_BYTES];
     TraceRec<TRACE> tr;
@@ -62,13 +74,13 @@ __global__ void __launch_bounds__(256) gemm_stream_kernel(const DecodeArgs p) {
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int col0 = blockIdx.x * 32;
+    const int col0 = blockIdx.x * BN;
     const int M = p.M, N = p.N, K = p.K;
     const int KT = K / 64;                                   // slabs (K % 64 == 0 is a launch precondition)
     const int cnt = (KT - wave + 3) / 4;                     // slabs of this wave: wave, wave+4, ...
 
     const int rowsA = M < BM ? M : BM;
-    const int rowsB = (N - col0) < 32 ? (N - col0) : 32;
+    const int rowsB = (N - col0) < BN ? (N - col0) : BN;
     const unsigned char* Ab = (const unsigned char*)p.A;
     const unsigned char* Bb = (const unsigned char*)p.B + (size_t)col0 * p.ldb * 2;
     const uint32_t bytesA = (uint32_t)((rowsA - 1) * p.lda + K) * 2u;
@@ -116,19 +128,24 @@ __global__ void __launch_bounds__(256) gemm_stream_kernel(const DecodeArgs p) {
         }
     };
 
-    // fragment reads: lane holds row (lane & 31), k chunk 2*ks + (lane >> 5).  With BM = 16
-    // the upper half of the A operand reads B rows: finite values that only reach rows of
-    // the accumulator that are never stored.
-    const int l32 = lane & 31, hi = lane >> 5;
-    int rd_off[4];
+    // fragment reads: lane holds row (lane % R), k chunk ks * 64 / R + lane / R.  With BN = 32 and
+    // BM = 16 the upper half of the A operand reads B rows, with BN = 8 the upper half of the B
+    // operand repeats the lower: values that only reach elements of the accumulator that are
+    // never stored.
+    const int lrow = lane % R, lh = lane / R;
+    const int lb = lrow < BN ? lrow : lrow - BN;                // (BN = 24, 8: the block's upper columns repeat the lower)
+    int rd_a[KS], rd_b[KS];
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) rd_off[ks] = l32 * 128 + ((((ks << 1) | hi) ^ swz(l32)) << 4);
+    for (int ks = 0; ks < KS; ++ks) {
+        rd_a[ks] = lrow * 128 + (((ks * (64 / R) + lh) ^ swz(lrow)) << 4);
+        rd_b[ks] = lb * 128 + (((ks * (64 / R) + lh) ^ swz(lb)) << 4);
+    }
 
-    f32x16_t acc[MI];
+    std::conditional_t<WIDE, f32x16_t, f32x4_t> acc[MI];
 #pragma unroll
     for (int a = 0; a < MI; ++a)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) acc[a][e] = 0.0f;
+        for (int e = 0; e < R * R / 64; ++e) acc[a][e] = 0.0f;
 
 #pragma unroll
     for (int i = 0; i < NS - 1; ++i) dma_slab(i, i);
@@ -142,17 +159,20 @@ __global__ void __launch_bounds__(256) gemm_stream_kernel(const DecodeArgs p) {
         tr.wait_end();
         dma_slab(i + NS - 1, s == 0 ? NS - 1 : s - 1);
         const unsigned char* st = ring + s * STAGE;
-        u32x4_t fa[MI][4], fb[4];
+        u32x4_t fa[MI][KS], fb[KS];
 #pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
+        for (int ks = 0; ks < KS; ++ks) {
 #pragma unroll
-            for (int a = 0; a < MI; ++a) fa[a][ks] = *(const u32x4_t*)(st + a * 4096 + rd_off[ks]);
-            fb[ks] = *(const u32x4_t*)(st + BM * 128 + rd_off[ks]);
+            for (int a = 0; a < MI; ++a) fa[a][ks] = *(const u32x4_t*)(st + a * R * 128 + rd_a[ks]);
+            fb[ks] = *(const u32x4_t*)(st + BM * 128 + rd_b[ks]);
         }
 #pragma unroll
-        for (int ks = 0; ks < 4; ++ks)
+        for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
-            for (int a = 0; a < MI; ++a) acc[a] = mfma_32x32x16<DT>(fb[ks], fa[a][ks], acc[a]);
+            for (int a = 0; a < MI; ++a) {
+                if constexpr (WIDE) acc[a] = mfma_32x32x16<DT>(fb[ks], fa[a][ks], acc[a]);
+                else acc[a] = mfma_16x16x32<DT>(fb[ks], fa[a][ks], acc[a]);
+            }
         s = s + 1 == NS ? 0 : s + 1;
     }
     // requests past K are still heading for the ring: drain before it is reused
@@ -160,23 +180,27 @@ __global__ void __launch_bounds__(256) gemm_stream_kernel(const DecodeArgs p) {
     tr.loop_end();
 
     // ---- add the four partial tiles in wave order, round, store ----
-    // lane holds P[m][n .. n+3], m = 32a + (lane & 31), n = 8g + 4*(lane >> 5)
+    // lane holds P[m][n .. n+3], m = R*a + lane % R, n = (256/R)*g + 4*(lane / R): the partial tile is
+    // MI*R rows of BN columns
     float* part = (float*)(lds + wave * RING);
 #pragma unroll
     for (int a = 0; a < MI; ++a)
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            float4 v = {acc[a][g * 4 + 0], acc[a][g * 4 + 1], acc[a][g * 4 + 2], acc[a][g * 4 + 3]};
-            *(float4*)(part + (a * 32 + l32) * 32 + g * 8 + hi * 4) = v;
+        for (int g = 0; g < R * R / 256; ++g) {
+            const float4 v = {acc[a][g * 4 + 0], acc[a][g * 4 + 1], acc[a][g * 4 + 2], acc[a][g * 4 + 3]};
+            const int n = g * (256 / R) + lh * 4;
+            if (BN >= R || n < BN) *(float4*)(part + (a * R + lrow) * BN + n) = v;
         }
     __syncthreads();
+    constexpr int RP = 256 / (BN / 4);                       // rows of C a pass of the 256 threads covers
 #pragma unroll
-    for (int a = 0; a < MI; ++a) {
-        const int m = a * 32 + (tid >> 3), n = (tid & 7) * 4;
-        float4 sum = *(const float4*)((const float*)lds + m * 32 + n);
+    for (int a = 0; a < (MI * R + RP - 1) / RP; ++a) {
+        const int m = a * RP + tid / (BN / 4), n = tid % (BN / 4) * 4;
+        if (tid >= RP * (BN / 4) || m >= MI * R) break;
+        float4 sum = *(const float4*)((const float*)lds + m * BN + n);
 #pragma unroll
         for (int w = 1; w < 4; ++w) {
-            const float4 v = *(const float4*)((const float*)(lds + w * RING) + m * 32 + n);
+            const float4 v = *(const float4*)((const float*)(lds + w * RING) + m * BN + n);
             sum.x += v.x; sum.y += v.y; sum.z += v.z; sum.w += v.w;
         }
         if (p.alpha != 1.0f || p.beta != 0.0f) {
@@ -197,8 +221,8 @@ __global__ void __launch_bounds__(256) gemm_stream_kernel(const DecodeArgs p) {
 
 template <class Cfg>
 hipError_t launch_stream_kernel(const DecodeArgs& a, hipStream_t stream) {
-    return a.DB ? launch_kernel(gemm_stream_kernel<Cfg, true>, dim3((a.N + 31) / 32), dim3(256), stream, a)
-                : launch_kernel(gemm_stream_kernel<Cfg, false>, dim3((a.N + 31) / 32), dim3(256), stream, a);
+    return a.DB ? launch_kernel(gemm_stream_kernel<Cfg, true>, dim3((a.N + Cfg::BN - 1) / Cfg::BN), dim3(256), stream, a)
+                : launch_kernel(gemm_stream_kernel<Cfg, false>, dim3((a.N + Cfg::BN - 1) / Cfg::BN), dim3(256), stream, a);
 }
 
 }  // namespace mi

@@ -86,7 +86,7 @@ class GemmTuner:
         self.param_space = {
             'KIND': ['mfma16', 'ring', 'ring16', 'tile', 'stream', 'decode', 'wavek'],
             'BM': [16, 32, 64, 96, 128, 192, 256],
-            'BN': [32, 64, 96, 128, 192, 256],
+            'BN': [32, 64, 96, 128, 192, 256, 8, 16, 24],
             'WM': [2, 4],
             'WN': [2, 4],
             'NS': [4, 1, 2, 3, 5],
@@ -114,7 +114,7 @@ class GemmTuner:
     def config_name(params: Dict[str, int]) -> str:
         c = dict({'OCC': 1, 'SWZ': 1, 'DTL': 1, 'EPI': 1}, **params)
         if c['KIND'] == 'stream':
-            c['BN'] = 32
+            c['BN'] = min(c.get('BN', 32), 32)
         return kc.config_name(c)
 
     def generate_code(self, params: Dict[str, int]) -> str:
@@ -169,7 +169,7 @@ class GemmTuner:
 
     # parameters that mean nothing for a kind: only their first value in the space is kept
     UNUSED = {'tile': ('NS', 'DRAIN', 'SHARED'), 'mfma16': ('NS', 'SHARED'), 'ring': ('DRAIN', 'OCC', 'SHARED'),
-              'ring16': ('DRAIN', 'OCC', 'SHARED'), 'stream': ('BN', 'WM', 'WN', 'GROUP', 'DRAIN', 'OCC', 'SHARED'),
+              'ring16': ('DRAIN', 'OCC', 'SHARED'), 'stream': ('WM', 'WN', 'GROUP', 'DRAIN', 'OCC', 'SHARED'),
               'decode': ('WM', 'WN', 'GROUP', 'DRAIN', 'OCC', 'SHARED'), 'wavek': ('WM', 'WN', 'GROUP', 'DRAIN', 'OCC')}
 
     def is_valid_configuration(self, params: Dict[str, int]) -> bool:
@@ -179,7 +179,14 @@ class GemmTuner:
             if key in params and key in self.param_space and params[key] != self.param_space[key][0]:
                 return False        # one copy of the configuration, not one per value of a parameter it ignores
         if c['KIND'] == 'stream':
-            c['BN'] = 32            # the single-pass decode kernel owns 32 columns per workgroup
+            # the single-pass decode kernel owns 8, 16, 24 or 32 columns per workgroup; the narrow ones are for few
+            # rows, with deep rings that leave room for a second workgroup (up to 21 KB a wave)
+            if c.get('BN', 32) > 32:
+                return False
+            if c.get('BN', 32) < 32 and (c['BM'] > 32 or c['NS'] < 3 or c['NS'] * (c['BM'] + c['BN']) > 168):
+                return False
+        elif c.get('BN', 32) < 32:
+            return False
         if c['KIND'] == 'wavek' and not c.get('SHARED'):
             c.pop('SHARED', None)
         try:

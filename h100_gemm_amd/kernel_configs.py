@@ -15,7 +15,8 @@ template takes (matmul_h100.cu.jinja:9-14) -- re-cast for CDNA4:
              "mfma16" / "ring16" (the same two pipelines on the 16x16x32 MFMA with eight
              or four waves, csrc/gemm_mfma16_kernel.hpp), "decode" (split-K kernel for decode
              shapes, M <= BM, whose LDS ring holds B only, csrc/gemm_decode_kernel.hpp) or
-             "stream" (single-pass decode kernel, csrc/gemm_stream_kernel.hpp), "wavek" (small
+             "stream" (single-pass decode kernel on BN = 8, 16, 24 or 32 columns a
+             workgroup, csrc/gemm_stream_kernel.hpp), "wavek" (small
              tiles with K split over the waves of a workgroup, or on a ring shared by them, for
              outputs of few tiles: any M, N and K, csrc/gemm_wavek_kernel.hpp)
     EPI      1: C tile transposed through LDS and written 16 bytes per lane, 0: 8-byte stores
@@ -108,7 +109,7 @@ def is_valid_config(c: dict) -> bool:
         del main["EWM"], main["EWN"]
         return is_valid_config(twin) and is_valid_config(main)
     if c["KIND"] == "stream":
-        return (c["BM"] in (16, 32, 64) and c["BN"] == 32 and c["NS"] >= 2
+        return (c["BM"] in (16, 32, 64) and c["BN"] in (8, 16, 24, 32) and c["NS"] >= 2
                 and (c["NS"] - 1) * ((c["BM"] + c["BN"]) // 8) <= 63
                 and c["NS"] * (c["BM"] + c["BN"]) * 128 >= max(c["BM"], 32) * 128
                 and lds_bytes(c) <= 160 * 1024)
@@ -220,8 +221,8 @@ def _q(BM, BN, WM, WN, NS=4, GROUP=4):
     return dict(KIND="ring16", BM=BM, BN=BN, WM=WM, WN=WN, NS=NS, GROUP=GROUP)
 
 
-def _s(BM, NS):
-    return dict(KIND="stream", BM=BM, BN=32, NS=NS)
+def _s(BM, NS, BN=32):
+    return dict(KIND="stream", BM=BM, BN=BN, NS=NS)
 
 
 def _k(BM, BN, NS, WK=None, OCC=1, SHARED=0, WK_RAGGED=None, WK_ODD=None):
@@ -294,6 +295,12 @@ CONFIGS = [
     # found by the tuner's sweep of the small-tile kinds at 512^3 (256 tiles, one per CU, eight K
     # units: too few to split over the waves); no time model, a tuned shape only
     _k(32, 32, NS=4, SHARED=1, OCC=4),
+    # single-pass decode kernels on fewer columns a workgroup: N up to 2048 / 4096 / 6144 in one round
+    _s(16, 5, BN=8),
+    _s(16, 5, BN=16),
+    _s(16, 4, BN=24),
+    _s(32, 3, BN=16),
+    _s(32, 3, BN=24),
 ]
 
 assert all(is_valid_config(c) for c in CONFIGS), [config_name(c) for c in CONFIGS if not is_valid_config(c)]
@@ -311,5 +318,7 @@ assert all(n in {config_name(c) for c in CONFIGS} for n in TUNED_SHAPES.values()
 # The kernels the automatic choice for decode shapes names (select_decode_kernel in
 # template/kernel_table.hpp.jinja, where the thresholds and the measurements behind them are).
 DECODE_KERNELS = {"stream16": "s16x32_n3", "stream32": "s32x32_n3", "stream64": "s64x32_n3",
+                  "stream16x8": "s16x8_n5", "stream16x16": "s16x16_n5", "stream16x24": "s16x24_n4",
+                  "stream32x16": "s32x16_n3", "stream32x24": "s32x24_n3",
                   "decode64": "d64x128_n4", "decode128": "d128x128_n3", "tile128x256": "m128x256_w2x2_g4_b1"}
 assert all(n in {config_name(c) for c in CONFIGS} for n in DECODE_KERNELS.values())
