@@ -447,14 +447,18 @@ Choice choose(int requested, int M, int N, int K, bool streamable, bool splittab
 //
 // With K % 64 != 0 the K loop of the 16x16x32 kernel runs at 0.69-0.83 of its rate on whole lines
 // (4095 x 6143 with K = 3073 / 3072: 180.7 / 124.6 us; 8191^3 941, 8191 x 8191 x 8192 725).  What
-// the copy saves grows with M*N*K: per product of extents 9e-10 us with tiles whose loads bound
-// the step (256x192: 6.5-8.9e-10; 192x192: 8-10.7e-10; 128x256: 11e-10), 3.2e-10 with the 256x256
-// tile, whose MFMAs hide part of the loads (2.8-4.4e-10), and a copy of one operand alone saves half
-// of that or less.  It costs its launch and 7.5e-7 us per element copied (5 TB/s).  None / A / B / both in us:
-// 4095x6143x3073 181 / 167 / 168 / 145, 3000^3 67 / 74 / 72 / 63, 2100x2100x9000 in two pieces
-// 109 / 118 / 116 / 99, 2048x28672x4100 454 / 408 / 488 / 457, 28672x2048x4100 482 / 500 / 454 / 463,
-// 8192x8192x8200 858 / 816 / 842 / 817; not worth it: 2048x2048x2049 29 / 35 / 34 / 32,
-// 4000x4000x600 31 / 37 / 40 / 39.
+// the copy saves grows with M*N*K and with the rows a tile loads for its area, less what its MFMAs
+// hide: in us per product of extents, 3.5e-10 with 256x256 tiles (measured 2.8-4.4e-10), 6.4e-10 with
+// 256x192 (5.9-8.9), 9.2e-10 with 192x192 (7.6-11.5), 12e-10 with 128x256 (11-15.8), 15e-10 with
+// 192x128 (14.7-18), 21e-10 with 128x128 (15.7-27); about half of it with a short K (below 2450;
+// 3200 where two workgroups on a CU hide each other's loads); less where CUs idle.  One operand
+// alone: 0.45 of it with 256x256 tiles, and with the others when the copied one is much the smaller
+// (9000x1024x9000 223 -> 189 by B; 3000^3 67 -> 74 by A).  It costs its launch and 7.5e-7 us per
+// element (5 TB/s).  None / A / B / both in us: 4095x6143x3073 181 / 167 / 168 / 145, 3000^3 67 / 74 / 72 / 63, 2100x2100x9000 in two
+// pieces 109 / 118 / 116 / 99, 2048x28672x4100 454 / 408 / 488 / 457, 28672x2048x4100 482 / 500 / 454 /
+// 463, 8192x8192x8200 858 / 816 / 842 / 817; none / both: 1435x3790x13542 229 / 173, 2485x1090x5883
+// 89 / 65; not worth it: 2000x2000x3001 39-47 / 41, 2048x2048x2049 29 / 32, 3333x3333x1111 36 / 44,
+// 854x3626x2574 32 / 39, 4000x4000x600 31 / 39.
 struct PackPlan {
     bool a, b;
     bool any() const { return a || b; }
@@ -467,13 +471,16 @@ PackPlan choose_packing(const Choice& c, int M, int N, int K) {
     PackPlan best{false, false};
     if (K % 64 == 0 || e.kind != mi::KIND_MFMA16 || e.kg > 1) return best;
     const double mnk = (double)M * N * K;
-    const bool square = e.BM == 256 && e.BN == 256;
+    double rate = 2.2e-7 * (1.0 / e.BM + 1.0 / e.BN - 0.0062);
+    if (K < (e.occ > 1 ? 3200 : 2450)) rate *= 0.55;
+    const double wgs = (double)((M + e.BM - 1) / e.BM) * ((N + e.BN - 1) / e.BN) * c.splits;
+    if (wgs < c.cus) rate *= std::sqrt(wgs / c.cus);
     double best_gain = 3.6e-11 * mnk;                        // 2 % of the launch at 1.1 PFLOP/s
     for (int which = 1; which <= 3; ++which) {
         const PackPlan p{(which & 1) != 0, (which & 2) != 0};
         if (p.bytes(M, N, K) > kMaxPackedBytes) continue;
-        const double saves = (which == 3 ? (square ? 3.2e-10 : 9.0e-10) : (square ? 1.6e-10 : 3.0e-10)) * mnk;
-        const double gain = saves - 4.0 - 7.5e-7 * ((p.a ? (double)M : 0.0) + (p.b ? (double)N : 0.0)) * K;
+        if (which != 3 && e.BM + e.BN < 512 && (p.a ? 6LL * M > N : 6LL * N > M)) continue;
+        const double gain = (which == 3 ? 1.0 : 0.45) * rate * mnk - 4.0 - 7.5e-7 * ((p.a ? (double)M : 0.0) + (p.b ? (double)N : 0.0)) * K;
         if (gain > best_gain) {
             best = p;
             best_gain = gain;

@@ -689,7 +689,7 @@ def test_caller_workspace_launches_on_two_streams(mi, orc):
 # A and B are copied to whole-line rows first (both; A alone; B alone; with K in pieces), and not: K % 64
 # of 1, 63 and 8, rows and columns at the edges of the tiles
 @pytest.mark.parametrize("M,N,K,copied", [(2817, 2819, 2753, "AB"), (2500, 3000, 2623, "AB"), (2560, 3072, 2568, "AB"),
-                                          (2048, 28672, 1089, "A"), (28673, 2049, 1096, "B"), (2100, 2100, 9001, "AB"),
+                                          (2048, 28672, 2561, "A"), (28673, 2049, 2568, "B"), (2100, 2100, 9001, "AB"),
                                           (1024, 1024, 1025, "")])
 def test_operands_copied_to_whole_lines_change_no_bit(mi, orc, M, N, K, copied):
     """With a ragged K a large launch copies its operands to rows on 128-byte lines in its workspace.
