@@ -66,8 +66,13 @@ class GemmParams:
 
 def runKernel(M: int, N: int, K: int, A, B, C, DB=None, stream=None) -> None:
     """bf16 GEMM with the library's choice of kernel (matmul_h100_optimal.cu:32-59)."""
-    L = _lib.load()
-    _lib.check(L.mi_gemm_bf16(M, N, K, _ptr(A), _ptr(B), _ptr(C), _ptr(DB), _stream(stream)))
+    if stream is not None:
+        stream = _stream(stream)
+    rc = (_lib._native or _lib.native()).bf16(M, N, K, A, B, C, DB, stream)
+    if rc is None:
+        rc = _lib.load().mi_gemm_bf16(M, N, K, _ptr(A), _ptr(B), _ptr(C), _ptr(DB), stream)
+    if rc:
+        _lib.check(rc)
 
 
 def run_kernel(kernel_num: int, M: int, N: int, K: int, A, B, C, DB=None, stream=None) -> None:
@@ -86,10 +91,17 @@ def gpu_gemm(params: GemmParams, config: int | str = MI_CONFIG_AUTO, dtype: int 
     if params.alpha != 1.0 or params.beta != 0.0:
         raise ValueError("gpu_gemm computes alpha = 1, beta = 0 only (as the reference's kernels do); "
                          "gemm_epilogue applies alpha and beta")
-    L = _lib.load()
-    config = _config_index(L, config)
-    _lib.check(L.mi_gemm_ex(config, dtype, params.M, params.N, params.K, _ptr(params.A),
-                            _ptr(params.B), _ptr(params.C), _ptr(DB), _stream(stream)))
+    if isinstance(config, str):
+        config = _config_index(_lib.load(), config)
+    if stream is not None:
+        stream = _stream(stream)
+    rc = (_lib._native or _lib.native()).ex(config, dtype, params.M, params.N, params.K, params.A, params.B, params.C, DB,
+                                            stream)
+    if rc is None:
+        rc = _lib.load().mi_gemm_ex(config, dtype, params.M, params.N, params.K, _ptr(params.A), _ptr(params.B),
+                                    _ptr(params.C), _ptr(DB), stream)
+    if rc:
+        _lib.check(rc)
 
 
 def _config_index(L, config) -> int:
@@ -108,16 +120,24 @@ def gemm_epilogue(params: GemmParams, config: int | str = MI_CONFIG_AUTO, dtype:
     reference's bf16 kernel writes, matmul_utils.cuh:529,545).  With ``workspace`` (a
     DeviceBuffer of at least ``workspace_bytes(...)`` bytes) split-K partial sums go there and
     the call allocates nothing, like the reference's launcher (matmul_h100_optimal.cu:32-59)."""
-    L = _lib.load()
+    if isinstance(config, str):
+        config = _config_index(_lib.load(), config)
+    if stream is not None:
+        stream = _stream(stream)
+    p, native = params, _lib._native or _lib.native()
     if workspace is not None:
-        _lib.check(L.mi_gemm_epilogue_ws(_config_index(L, config), dtype, params.M, params.N, params.K,
-                                         _ptr(params.A), _ptr(params.B), _ptr(params.C), params.alpha,
-                                         params.beta, c_layout, workspace.ptr, workspace.nbytes,
-                                         _stream(stream)))
-        return
-    _lib.check(L.mi_gemm_epilogue(_config_index(L, config), dtype, params.M, params.N, params.K,
-                                  _ptr(params.A), _ptr(params.B), _ptr(params.C), params.alpha,
-                                  params.beta, c_layout, _stream(stream)))
+        rc = native.epilogue_ws(config, dtype, p.M, p.N, p.K, p.A, p.B, p.C, p.alpha, p.beta, c_layout, workspace.ptr,
+                                workspace.nbytes, stream)
+        if rc is None:
+            rc = _lib.load().mi_gemm_epilogue_ws(config, dtype, p.M, p.N, p.K, _ptr(p.A), _ptr(p.B), _ptr(p.C), p.alpha,
+                                                 p.beta, c_layout, workspace.ptr, workspace.nbytes, stream)
+    else:
+        rc = native.epilogue(config, dtype, p.M, p.N, p.K, p.A, p.B, p.C, p.alpha, p.beta, c_layout, stream)
+        if rc is None:
+            rc = _lib.load().mi_gemm_epilogue(config, dtype, p.M, p.N, p.K, _ptr(p.A), _ptr(p.B), _ptr(p.C), p.alpha,
+                                              p.beta, c_layout, stream)
+    if rc:
+        _lib.check(rc)
 
 
 def workspace_bytes(M: int, N: int, K: int, config: int | str = MI_CONFIG_AUTO, dtype: int = MI_DTYPE_BF16,
@@ -131,10 +151,15 @@ def reference_gpu_gemm(params: GemmParams, dtype: int = MI_DTYPE_BF16, stream=No
     """reference_gpu_gemm(GemmParams) of reference.h:78-90: the plain ascending-k GPU GEMM
     the harness uses as golden; honours alpha and beta (beta is a scalar added to every
     element, as in reference.h:40,72)."""
-    L = _lib.load()
-    _lib.check(L.mi_reference_gpu_gemm(dtype, params.M, params.N, params.K, _ptr(params.A),
-                                       _ptr(params.B), _ptr(params.C), params.alpha, params.beta,
-                                       _stream(stream)))
+    if stream is not None:
+        stream = _stream(stream)
+    p = params
+    rc = (_lib._native or _lib.native()).reference(dtype, p.M, p.N, p.K, p.A, p.B, p.C, p.alpha, p.beta, stream)
+    if rc is None:
+        rc = _lib.load().mi_reference_gpu_gemm(dtype, p.M, p.N, p.K, _ptr(p.A), _ptr(p.B), _ptr(p.C), p.alpha, p.beta,
+                                               stream)
+    if rc:
+        _lib.check(rc)
 
 
 # ---- config table --------------------------------------------------------------------

@@ -5,10 +5,13 @@ There is no fallback: if the shared library has not been built, loading raises.
 from __future__ import annotations
 
 import ctypes as C
+import importlib.machinery
+import importlib.util
 from pathlib import Path
 
 PKG = Path(__file__).resolve().parent
 LIB_PATH = PKG / "lib" / "libmi_gemm.so"
+PY_CALL_PATH = PKG / "lib" / "mi_py_call.so"
 
 MI_OK = 0
 MI_ERR_INVALID = -1
@@ -98,6 +101,28 @@ def load() -> C.CDLL:
         fn.argtypes = args
     _lib = L
     return L
+
+
+_native = None
+
+
+def native():
+    """The launching calls without ctypes (csrc/py_call.c, linked to the library): each takes the C
+    function's arguments, operands as the package's entry points take them, and returns its status, or
+    None -- nothing done -- when an argument is not of a usual kind and ctypes has to convert it."""
+    global _native
+    if _native is None:
+        load()
+        if not PY_CALL_PATH.exists():
+            raise ImportError(f"{PY_CALL_PATH} is missing: build it with `python -m h100_gemm_amd.build`. "
+                              "There is no fallback path.")
+        loader = importlib.machinery.ExtensionFileLoader("mi_py_call", str(PY_CALL_PATH))
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("mi_py_call", loader))
+        loader.exec_module(module)
+        from . import DeviceBuffer
+        module.set_device_buffer(DeviceBuffer)
+        _native = module
+    return _native
 
 
 def check(rc: int) -> None:

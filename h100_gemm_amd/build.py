@@ -13,6 +13,7 @@ import hashlib
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
@@ -25,6 +26,7 @@ PKG = Path(__file__).resolve().parent
 CSRC = PKG / "csrc"
 GEN = CSRC / "gen"
 LIB = PKG / "lib" / "libmi_gemm.so"
+PY_CALL = PKG / "lib" / "mi_py_call.so"
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 # -packed-fp32-ops off: packed fp32 VALU forms are not to be generated on this hardware pool.
@@ -130,6 +132,16 @@ def _compile(src: Path, force: bool) -> Path:
     return obj
 
 
+def build_py_call() -> Path:
+    """The package's launching calls as a CPython module beside the library (host code, linked to it)."""
+    cmd = ["gcc", "-O2", "-std=c11", "-Wall", "-shared", "-fPIC", f"-I{sysconfig.get_paths()['include']}",
+           str(CSRC / "py_call.c"), "-o", str(PY_CALL), f"-L{LIB.parent}", "-l:" + LIB.name, "-Wl,-rpath,$ORIGIN"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"gcc failed for py_call.c:\n{r.stderr[-4000:]}")
+    return PY_CALL
+
+
 def build(jobs: int | None = None, force: bool = False, verbose: bool = True) -> Path:
     units = render_sources()
     srcs = units + [CSRC / "mi_gemm.hip", CSRC / "reference_gpu_gemm.hip"]
@@ -141,6 +153,7 @@ def build(jobs: int | None = None, force: bool = False, verbose: bool = True) ->
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"link failed:\n{r.stderr[-4000:]}")
+    build_py_call()
     if verbose:
         print(f"built {LIB} ({LIB.stat().st_size} bytes, {len(units)} kernel configs)")
     return LIB

@@ -432,3 +432,52 @@ def test_automatic_choice_always_names_a_kernel_that_can_run_the_shape(mi):
         assert mi.select_config(M, N, K) == c
         picks.add(kc.CONFIGS[c]["KIND"])
     assert picks >= {"mfma16", "stream", "decode", "wavek"}
+
+
+def test_launching_calls_take_the_usual_arguments_and_leave_the_others_to_ctypes(mi):
+    """The C functions behind the package's entry points: ints within 32 bits, floats, operands as
+    None, int, DeviceBuffer or anything with data_ptr(), streams as None or int.  Anything else is None,
+    nothing done, and the entry point then raises what ctypes and the wrapper raise."""
+    class Operand:
+        def __init__(self, address):
+            self.address = address
+
+        def data_ptr(self):
+            return self.address
+
+    class Broken:
+        def data_ptr(self):
+            raise RuntimeError("no storage")
+
+    n = mi._lib.native()
+    bad = mi._lib.MI_ERR_INVALID
+    buf = object.__new__(mi.DeviceBuffer)
+    buf.ptr, buf.nbytes = 64, 64
+    for A in (64, Operand(64), buf, Operand(2**64 - 64)):
+        # (refused for M = 0 before any operand is looked at)
+        assert n.bf16(0, 8, 8, A, A, A, None, None) == bad and n.bf16(0, 8, 8, A, A, A, A, 64) == bad
+        assert n.ex(-1, 0, 0, 8, 8, A, A, A, None, None) == bad
+        assert n.epilogue(-1, 0, 0, 8, 8, A, A, A, 1.0, 0.0, 0, None) == bad
+        assert n.epilogue_ws(-1, 0, 0, 8, 8, A, A, A, 1.0, 0.0, 0, 64, 64, None) == bad
+        assert n.reference(0, 0, 8, 8, A, A, A, 1.0, 0.0, None) == bad
+    for A in (None, 0, Operand(0)):
+        assert n.bf16(8, 8, 8, A, 64, 64, None, None) == bad
+        assert b"null" in mi._lib.load().mi_last_error()
+    buf.ptr = 0                                              # (nothing to free)
+    for M in (8.0, 2**31, -2**31 - 1, True, "8", None):
+        assert n.bf16(M, 8, 8, 64, 64, 64, None, None) is None
+    for A in ("x", 1.0, -1, 2**64, Broken(), object()):
+        assert n.bf16(0, 8, 8, A, 64, 64, None, None) is None
+    assert n.bf16(0, 8, 8, 64, 64, 64, None, "stream") is None and n.bf16(0, 8, 8) is None
+    assert n.epilogue(-1, 0, 0, 8, 8, 64, 64, 64, 1, 0.0, 0, None) is None          # alpha an int
+    assert n.epilogue_ws(-1, 0, 0, 8, 8, 64, 64, 64, 1.0, 0.0, 0, 64, -1, None) is None
+    with pytest.raises(TypeError):
+        mi.runKernel(8, 8, 8, "x", 64, 64)
+    with pytest.raises(TypeError):
+        mi.runKernel(8, 8, 8, 64, 64, 64, stream="s")
+    with pytest.raises(RuntimeError, match="no storage"):
+        mi.runKernel(8, 8, 8, Broken(), 64, 64)
+    with pytest.raises(ctypes.ArgumentError):
+        mi.runKernel(8.0, 8, 8, 64, 64, 64)
+    with pytest.raises(mi.MiGemmError, match="positive"):
+        mi.gemm_epilogue(mi.GemmParams(0, 8, 8, 64, 64, 64, 2, 0))                   # an int alpha, as before
