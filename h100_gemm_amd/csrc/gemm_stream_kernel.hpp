@@ -8,7 +8,7 @@
 //     ~26 GB/s whatever it keeps in flight, so BN is the narrowest that keeps N / BN workgroups
 //     within one round of the CUs (stream_time_us in the kernel table): 1 x 4096 x 4096 with 32
 //     columns on 128 workgroups 9.2 us (3.6 TB/s), with 16 on 256 7.1 (4.7); 1 x 2048 x 4096 with 8
-//     5.2, 16 x 6144 x 4096 with 24 10.2 (32: 11.3).  Narrower still reads more of A, which every
+//     5.4, 16 x 6144 x 4096 with 24 10.2 (32: 11.3).  Narrower still reads more of A, which every
 //     workgroup walks whole: 16 x 8192 x 8192 with 32 21.9 us, with 16 24.0, with 8 30.2;
 //   * its four waves split K between them, 64-deep slab by slab (wave w takes slabs
 //     w, w+4, ...), so the workgroup as a whole walks 512 contiguous bytes of every row;

@@ -472,7 +472,7 @@ PackPlan choose_packing(const Choice& c, int M, int N, int K) {
     if (K % 64 == 0 || e.kind != mi::KIND_MFMA16 || e.kg > 1) return best;
     const double mnk = (double)M * N * K;
     double rate = 2.2e-7 * (1.0 / e.BM + 1.0 / e.BN - 0.0062);
-    if (K < (e.occ > 1 ? 3200 : 2450)) rate *= 0.55;
+    if (K < (e.occ > 1 ? 3200 : 2450)) rate *= 0.5;
     const double wgs = (double)((M + e.BM - 1) / e.BM) * ((N + e.BN - 1) / e.BN) * c.splits;
     if (wgs < c.cus) rate *= std::sqrt(wgs / c.cus);
     double best_gain = 3.6e-11 * mnk;                        // 2 % of the launch at 1.1 PFLOP/s

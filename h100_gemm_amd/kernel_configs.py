@@ -37,8 +37,12 @@ template takes (matmul_h100.cu.jinja:9-14) -- re-cast for CDNA4:
              tiles per CU with a K too short to split four ways, or tiles too large for that
     WK       (wavek, optional) time model in microseconds, (fixed, per round, per unit, per
              tile): fixed + rounds of co-resident workgroups (tiles / (CUs x OCC), rounded up)
-             x per round + tiles per CU (rounded up) x (per tile + K/64 x per unit);
-             non-negative least squares on 89-99 shapes (the 96x64 shared-ring config: x 1.035); configs that carry it join the automatic choice
+             x per round + tiles per CU (rounded up) x (per tile + K/64 x per unit); robust
+             non-negative least squares on up to 620 shapes of the small and middle range, A and B
+             coming from memory (rotated through 500 MB; over operands that stay in the caches
+             the units are 15-25 % shorter and the private rings' lead over the shared one with a
+             long K does not show: 896x1536x3712 on 96x64 20.5 / 25.4 us); 6.5-8.6 % mean error;
+             configs that carry it join the automatic choice
     WK_RAGGED (wavek, optional) what a K unit costs more when K % 64 != 0 (rows that do not start on
              128-byte lines): K % 8 == 0 with K < 2048 / K >= 2048, other even K with K < 2048 /
              K >= 2048 (medians over 160 shapes of four lists); WK_ODD the same for an odd K
@@ -281,16 +285,16 @@ CONFIGS = [
     _m(128, 128, 2, 2, DRAIN=1, KG=2, EFF=0.64, EFF_E=0.93),
     _d(128, NS=3),
     _d(64, NS=4),
-    _k(32, 32, NS=1, OCC=5, WK=(2.18, 0.0, 0.0775, 0.314), WK_RAGGED=(1.26, 1.40, 1.46, 1.48), WK_ODD=1.95),
-    _k(32, 32, NS=2, OCC=2, WK=(1.71, 0.153, 0.0753, 0.580), WK_RAGGED=(1.19, 1.43, 1.55, 1.49), WK_ODD=1.97),
-    _k(64, 32, NS=3, WK=(0.87, 2.10, 0.1188, 0.0), WK_RAGGED=(1.21, 1.49, 1.83, 1.71), WK_ODD=2.05),
-    _k(64, 64, NS=1, OCC=2, WK=(1.93, 2.19, 0.1792, 0.0), WK_RAGGED=(1.00, 1.35, 1.34, 1.51), WK_ODD=1.70),
-    _k(64, 64, NS=2, WK=(0.88, 2.81, 0.1648, 0.0), WK_RAGGED=(1.11, 1.49, 1.67, 1.69), WK_ODD=1.97),
-    _k(96, 64, NS=2, WK=(1.35, 4.06, 0.2306, 0.0), WK_RAGGED=(0.85, 1.27, 1.25, 1.45), WK_ODD=1.73),
-    _k(96, 96, NS=4, SHARED=1, WK=(1.03, 3.336, 0.3179, 0.0), WK_RAGGED=(0.98, 1.24, 1.16, 1.37), WK_ODD=1.58),
-    _k(64, 64, NS=4, SHARED=1, OCC=2, WK=(1.31, 1.734, 0.1815, 0.0), WK_RAGGED=(1.06, 1.44, 1.31, 1.60), WK_ODD=1.77),
-    _k(96, 64, NS=4, SHARED=1, OCC=2, WK=(1.96, 1.90, 0.2313, 0.217), WK_RAGGED=(0.98, 1.32, 1.21, 1.52), WK_ODD=1.72),
-    _k(64, 32, NS=4, SHARED=1, OCC=3, WK=(1.54, 1.362, 0.1234, 0.0), WK_RAGGED=(1.20, 1.49, 1.49, 1.64), WK_ODD=1.92),
+    _k(32, 32, NS=1, OCC=5, WK=(2.71, 0.000, 0.0963, 0.155), WK_RAGGED=(1.12, 1.27, 1.28, 1.44), WK_ODD=1.73),
+    _k(32, 32, NS=2, OCC=2, WK=(2.43, 0.000, 0.0901, 0.598), WK_RAGGED=(1.08, 1.27, 1.43, 1.43), WK_ODD=1.81),
+    _k(64, 32, NS=3, WK=(1.64, 1.943, 0.1441, 0.168), WK_RAGGED=(1.16, 1.36, 1.66, 1.57), WK_ODD=1.96),
+    _k(64, 64, NS=1, OCC=2, WK=(2.88, 0.000, 0.1980, 0.885), WK_RAGGED=(1.19, 1.31, 1.51, 1.47), WK_ODD=1.75),
+    _k(64, 64, NS=2, WK=(1.55, 2.600, 0.1900, 0.0), WK_RAGGED=(1.19, 1.36, 1.63, 1.51), WK_ODD=1.88),
+    _k(96, 64, NS=2, WK=(1.45, 3.322, 0.2531, 0.017), WK_RAGGED=(1.18, 1.36, 1.65, 1.48), WK_ODD=1.87),
+    _k(96, 96, NS=4, SHARED=1, WK=(0.68, 2.653, 0.3857, 0.140), WK_RAGGED=(1.17, 1.44, 1.41, 1.44), WK_ODD=1.67),
+    _k(64, 64, NS=4, SHARED=1, OCC=2, WK=(1.99, 0.882, 0.2289, 0.000), WK_RAGGED=(1.23, 1.31, 1.43, 1.39), WK_ODD=1.68),
+    _k(96, 64, NS=4, SHARED=1, OCC=2, WK=(1.85, 1.299, 0.2848, 0.000), WK_RAGGED=(1.24, 1.49, 1.47, 1.67), WK_ODD=1.76),
+    _k(64, 32, NS=4, SHARED=1, OCC=3, WK=(2.66, 0.131, 0.1614, 0.000), WK_RAGGED=(1.21, 1.35, 1.43, 1.54), WK_ODD=1.75),
     _m(192, 256, 2, 2, DRAIN=1, EFF=0.89, EFF_E=0.92),
     # found by the tuner's sweep of the small-tile kinds at 512^3 (256 tiles, one per CU, eight K
     # units: too few to split over the waves); no time model, a tuned shape only
