@@ -4,7 +4,7 @@
 // tiled kernels load straddle two cache lines, and each line is fetched by two consecutive K
 // steps; the K loop then runs at 0.69-0.83 of its rate on whole lines.  The copy reads each
 // operand once and writes it once; past a certain size that is less than what it saves (the rule
-// is packing_pays in mi_gemm.hip).  Rows are padded with zeros to a whole number of 64-deep slabs:
+// is choose_packing in mi_gemm.hip).  Rows are padded with zeros to a whole number of 64-deep slabs:
 // zero products at the end of every sum, so C is bit for bit the same.
 #pragma once
 
