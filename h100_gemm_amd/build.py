@@ -63,7 +63,8 @@ def render_sources(configs=None) -> list[Path]:
                                      tuned=[(m, n, k, [c["name"] for c in named].index(nm))
                                             for (m, n, k), nm in sorted(getattr(kc, "TUNED_SHAPES", {}).items())
                                             if nm in [c["name"] for c in named]],
-                                     decode_idx=_decode_indices(named)))
+                                     decode_idx=_decode_indices(named),
+                                     deep_twin=[c["name"] for c in named].index(kc.DEEP_TWIN)))
     # drop units of configs that no longer exist
     keep = {p.name for p in units}
     for old in GEN.glob("unit_*.hip"):
@@ -104,6 +105,9 @@ def check_text(name: str, text: str) -> None:
     # {bf16, fp16} x {aligned, predicated} x {plain, trace} for the 16x16x32 kernel (and as many again
     # with K cut over workgroups, where the config does not split K over groups of its waves)
     isa_check.check_m0(name, text, need_kernels=8 if cfg["KIND"] == "mfma16" else 1)
+    if cfg.get("DEEP"):                         # {bf16, fp16} x {whole K, whole lines} x {plain, split-K}, traced and not
+        if isa_check.check_no_scratch(name, text, r"gemm_deep_kernel") != 16:
+            raise RuntimeError(f"{name}: deep-ring kernels are missing from the assembly text")
     if cfg["KIND"] == "mfma16" and cfg.get("EFF"):
         isa_check.check_no_scratch(name, text)
     isa_check.check_lds_bytes(name, text, kc.lds_bytes(cfg))

@@ -134,6 +134,23 @@ int choose_small_tile_splits(const mi::KernelEntry& e, int M, int N, int K, bool
     return mi::best_wavek_splits(e, M, N, K, true, cus, k_per_split, nullptr);
 }
 
+// Split-K for the deep-ring kernels, as for the tiled one (MI_GEMM_TILE_SPLITK forces a piece count here too).
+int choose_deep_splits(const mi::KernelEntry& e, int M, int N, int K, bool splittable, int cus, int* k_per_split) {
+    *k_per_split = K;
+    static const int env = [] { const char* s = getenv("MI_GEMM_TILE_SPLITK"); return s ? atoi(s) : 0; }();
+    if (!splittable || env == 1) return 1;
+    if (env > 1) {
+        int s = env < K / 512 ? env : K / 512;
+        if (s < 2 || (long long)M * N * 4 >= 0x7fffffffLL) return 1;
+        const int kps = ((K + s - 1) / s + 127) / 128 * 128;
+        s = (K + kps - 1) / kps;
+        if (s < 2) return 1;
+        *k_per_split = kps;
+        return s;
+    }
+    return mi::best_deep_splits(e, M, N, K, true, cus, k_per_split, nullptr);
+}
+
 // ---- where the split-K kernels put their fp32 partial sums ----------------------------
 // Three sources, chosen by the entry point:
 //  * LIBRARY (mi_gemm_bf16 / _ex / _epilogue): one buffer per (device, stream) -- and thread, for
@@ -476,12 +493,13 @@ const std::vector<TunedEntry>& tuned_entries() {
     return table;
 }
 // config for (M, N, K) from the tuned file, or -1
-int tuned_config(int M, int N, int K, bool streamable, bool small_ok) {
+int tuned_config(int M, int N, int K, bool streamable, bool ptr_aligned, bool small_ok) {
     for (const TunedEntry& t : tuned_entries()) {
         if (t.M != M || t.N != N || t.K != K) continue;
         const mi::KernelEntry& e = mi::kKernels[t.config];
         if ((is_split_k_decode(e.kind) || e.kind == mi::KIND_STREAM) && (!streamable || M > e.BM)) continue;
         if (e.kind == mi::KIND_WAVEK && !small_ok) continue;
+        if (e.kind == mi::KIND_DEEP && !mi::deep_runs(K, ptr_aligned)) continue;
         if (e.kg > 1 && K % (128 * e.kg) != 0) continue;      // (the rule mi_gemm_config_supports applies)
         return t.config;
     }
@@ -495,18 +513,24 @@ int tuned_config(int M, int N, int K, bool streamable, bool small_ok) {
 struct Choice {
     int M, N, K, flags, requested, cus;   // key; requested = the caller's config (MI_CONFIG_AUTO or an index)
     int config, splits, k_per_split;
+    bool deep;                            // the config's deep-ring kernel runs the call
 };
 Choice compute_choice(int requested, int M, int N, int K, bool streamable, bool splittable, bool ptr_aligned,
                       bool small_ok) {
     const int flags = (streamable ? 1 : 0) | (splittable ? 2 : 0) | (ptr_aligned ? 4 : 0) | (small_ok ? 8 : 0);
     const int cus = compute_units();
-    Choice c{M, N, K, flags, requested, cus, requested, 1, K};
+    Choice c{M, N, K, flags, requested, cus, requested, 1, K, false};
     if (requested == MI_CONFIG_AUTO) {
-        c.config = tuned_config(M, N, K, streamable, small_ok);
+        c.config = tuned_config(M, N, K, streamable, ptr_aligned, small_ok);
         if (c.config < 0) c.config = mi::select_kernel(M, N, K, streamable, splittable, ptr_aligned, small_ok, cus);
     }
+    // (a config that has only a deep-ring kernel runs what that cannot on 128x128 tiles)
+    if (mi::kKernels[c.config].kind == mi::KIND_DEEP && !mi::deep_runs(K, ptr_aligned)) c.config = mi::kDeepTwin;
     const mi::KernelEntry& e = mi::kKernels[c.config];
-    if (e.kind == mi::KIND_MFMA16) {
+    c.deep = e.deep[0][0] && K <= e.deep_max_k && mi::deep_runs(K, ptr_aligned);
+    if (c.deep) {
+        c.splits = choose_deep_splits(e, M, N, K, splittable, cus, &c.k_per_split);
+    } else if (e.kind == mi::KIND_MFMA16) {
         c.splits = choose_tile_splits(e, M, N, K, splittable, ptr_aligned, cus, &c.k_per_split);
     } else if (is_split_k_decode(e.kind) && streamable && M <= e.BM) {
         const int tiles_n = (N + e.BN - 1) / e.BN;
@@ -572,7 +596,7 @@ struct PackPlan {
 PackPlan choose_packing(const Choice& c, int M, int N, int K) {
     const mi::KernelEntry& e = mi::kKernels[c.config];
     PackPlan best{false, false};
-    if (K % 64 == 0 || e.kind != mi::KIND_MFMA16 || e.kg > 1) return best;
+    if (K % 64 == 0 || e.kind != mi::KIND_MFMA16 || e.kg > 1 || c.deep) return best;
     const double mnk = (double)M * N * K;
     double rate = 2.2e-7 * (1.0 / e.BM + 1.0 / e.BN - 0.0062);
     if (K < (e.occ > 1 ? 3200 : 2450)) rate *= 0.5;
@@ -627,7 +651,7 @@ int run_gemm(int config, int dtype, int M, int N, int K, const void* A, const vo
     if (rc != MI_OK) return rc;
     const bool streamable = shape_is_streamable(M, N, K, A, B, C);
     if (may_cut && config == MI_CONFIG_AUTO &&
-        tuned_config(M, N, K, streamable, shape_has_word_rows(K, A, B)) < 0) {       // (a tuned shape runs as tuned)
+        tuned_config(M, N, K, streamable, aligned16(A) && aligned16(B) && aligned16(C), shape_has_word_rows(K, A, B)) < 0) {       // (a tuned shape runs as tuned)
         const int m1 = rows_to_cut(M, N, K, streamable, shape_is_splittable(N, C),
                                    aligned16(A) && aligned16(B) && aligned16(C), shape_has_word_rows(K, A, B));
         if (m1 > 0) {
@@ -698,7 +722,7 @@ int run_gemm(int config, int dtype, int M, int N, int K, const void* A, const vo
             return fail(MI_ERR_HIP, "launch of %s failed: %s", e.name, hipGetErrorString(err));
         return MI_OK;
     }
-    if (e.kind == mi::KIND_WAVEK) {
+    if (e.kind == mi::KIND_WAVEK && !choice.deep) {
         if (!shape_has_word_rows(K, A, B))
             return fail(MI_ERR_UNSUPPORTED, "config %s needs 4-byte aligned A and B", e.name);
         args.splits = choice.splits;
@@ -742,7 +766,7 @@ int run_gemm(int config, int dtype, int M, int N, int K, const void* A, const vo
     if (e.kg > 1 && K % (128 * e.kg) != 0)
         return fail(MI_ERR_UNSUPPORTED, "config %s splits K over %d groups of waves and needs K %% %d == 0", e.name,
                     e.kg, 128 * e.kg);
-    if (e.kind == mi::KIND_MFMA16) {
+    if (e.kind == mi::KIND_MFMA16 || choice.deep) {
         args.splits = choice.splits;
         args.k_per_split = choice.k_per_split;
         const size_t split_bytes = args.splits > 1 ? (size_t)args.splits * M * N * sizeof(float) : 0;
@@ -792,8 +816,8 @@ int run_gemm(int config, int dtype, int M, int N, int K, const void* A, const vo
         }
         if (args.splits == 1) args.k_per_split = args.K;
     }
-    const bool edge = !shape_is_aligned(e, M, N, args.K, args.A, args.B, C);
-    mi::LaunchFn fn = e.launch[dtype][edge ? 1 : 0];
+    const bool edge = choice.deep ? K % 64 != 0 : !shape_is_aligned(e, M, N, args.K, args.A, args.B, C);
+    mi::LaunchFn fn = choice.deep ? e.deep[dtype][edge ? 1 : 0] : e.launch[dtype][edge ? 1 : 0];
     if (!fn) return fail(MI_ERR_UNSUPPORTED, "config %s has no %s kernel for dtype %d", e.name,
                          edge ? "predicated" : "aligned", dtype);
     hipError_t err = fn(args, (hipStream_t)stream);
@@ -847,7 +871,7 @@ int mi_gemm_config_supports(int config, int dtype, int M, int N, int K) {
         return M <= e.BM && N % 4 == 0 && K % 64 == 0;
     if (e.kind == mi::KIND_WAVEK) return 1;
     if (e.kg > 1 && K % (128 * e.kg) != 0) return 0;
-    return e.launch[dtype][1] != nullptr;
+    return e.kind == mi::KIND_DEEP || e.launch[dtype][1] != nullptr;
 }
 
 int mi_gemm_config_grid(int config, int M, int N, int K) {
@@ -860,6 +884,10 @@ int mi_gemm_config_grid(int config, int M, int N, int K) {
         return tiles_n * choose_splits(tiles_n, K, compute_units());
     }
     const int tiles = ((M + e.BM - 1) / e.BM) * ((N + e.BN - 1) / e.BN);
+    if (e.deep[0][0] && K <= e.deep_max_k && mi::deep_runs(K, true)) {
+        int kps = K;
+        return tiles * choose_deep_splits(e, M, N, K, N % 4 == 0, compute_units(), &kps);
+    }
     if (e.kind == mi::KIND_WAVEK) {    // split-K pieces, assuming an aligned C and no trace buffer
         int kps = K;
         return tiles * choose_small_tile_splits(e, M, N, K, N % 4 == 0, compute_units(), &kps);
@@ -876,7 +904,7 @@ int mi_gemm_select_config(int dtype, int M, int N, int K) {
     if (!shape_in_range(M, N, K)) return -1;
     // pointer alignment is unknown here: assume the usual 256-byte aligned allocations
     const bool streamable = N % 4 == 0 && K % 64 == 0;
-    const int tuned = tuned_config(M, N, K, streamable, true);
+    const int tuned = tuned_config(M, N, K, streamable, true, true);
     if (tuned >= 0) return tuned;
     return mi::select_kernel(M, N, K, streamable, N % 4 == 0, true, true, compute_units());
 }
@@ -885,7 +913,7 @@ int mi_gemm_row_cut(int dtype, int M, int N, int K) {
     (void)dtype;
     if (!shape_in_range(M, N, K)) return 0;
     const bool streamable = N % 4 == 0 && K % 64 == 0;
-    if (tuned_config(M, N, K, streamable, true) >= 0) return 0;
+    if (tuned_config(M, N, K, streamable, true, true) >= 0) return 0;
     return rows_to_cut(M, N, K, streamable, N % 4 == 0, true, true);
 }
 
@@ -962,7 +990,7 @@ size_t mi_gemm_workspace_bytes(int config, int dtype, int M, int N, int K, int c
         return need;
     };
     size_t need = uncut(M);
-    if (config == MI_CONFIG_AUTO && tuned_config(M, N, K, N % 4 == 0 && K % 64 == 0, true) < 0)
+    if (config == MI_CONFIG_AUTO && tuned_config(M, N, K, N % 4 == 0 && K % 64 == 0, true, true) < 0)
         for (int flags = 0; flags < 16; ++flags) {
             const int m1 = rows_to_cut(M, N, K, (flags & 1) != 0 && N % 4 == 0 && K % 64 == 0, (flags & 2) != 0 && N % 4 == 0,
                                        (flags & 4) != 0, (flags & 8) != 0);

@@ -287,6 +287,61 @@ def test_k_groups_inside_the_workgroup(mi, orc, config):
         assert (guard == 0xEEEE).all(), "bytes outside C were written"
 
 
+def deep_configs():
+    from h100_gemm_amd import kernel_configs as kc
+    return [i for i, c in enumerate(kc.CONFIGS) if c.get("DEEP") and c.get("KG", 1) == 1]
+
+
+@pytest.mark.parametrize("config", deep_configs())
+def test_deep_ring_kernels(mi, orc, config):
+    """The deep ring of whole lines: K around every count of slabs the ring, its plain trips and its last trips make
+    (K % 64 of 0, 8 and 56), M and N around the tile, operands at 16-byte phases of a line, K in pieces with a ragged
+    last one, alpha / beta and column-major C.  Integer fills: any order of sums gives the oracle's bits."""
+    from h100_gemm_amd import kernel_configs as kc
+    c = kc.CONFIGS[config]
+    bm, bn, ns, top = c["BM"], c["BN"], c["DEEP"], c.get("DEEP_MAX_K", 1 << 30)
+    for k in (2, ns - 1, ns, 2 * ns, 2 * ns + 1, 3 * ns + 1):
+        for K in (64 * k - 8, 64 * k, 64 * k + 8):
+            if 128 <= K <= top:
+                check(mi, orc, bm + 1, bn - 3, K, "int", config=config, exact=True)
+    for M, N, K in [(1, 1, 128), (2 * bm, 2 * bn, 256), (bm - 1, 2 * bn + 1, 200), (3 * bm + 5, 7, 648), (5, 300, 712)]:
+        check(mi, orc, M, N, K, "int", config=config, exact=True)
+    rng = np.random.default_rng(7)
+    for phase in range(8):
+        K = 8 * int(rng.integers(16, 100))
+        C, ref, guard = _run_offset(mi, orc, config, bm + 9, bn + 6, K, 16 * (phase & 3), 32 * (phase >> 2), 16 * (phase & 3))
+        assert (C == ref).all() and (guard == 0xEEEE).all(), (phase, K)
+    check(mi, orc, 300, 517, min(top, 1000), "uniform", config=config)
+    check(mi, orc, 517, 300, min(top, 1024), "normal", config=config, dtype=orc.FP16)
+    check_epilogue(mi, orc, 300, 260, 968, "int", -0.5, 2.75, config=config, exact=True)
+    check_epilogue(mi, orc, 200, 131, 1024, "int", 2.0, -1.0, config=config, c_layout=mi.MI_C_COL_MAJOR, exact=True)
+    if top > 8192:
+        assert mi.config_grid(config, 2 * bm, 2 * bn, 8200) > 4                 # K in pieces
+        for K in (8192, 8200, 4104):
+            check(mi, orc, 2 * bm - 1, 2 * bn, K, "int", config=config, exact=True)
+        check(mi, orc, bm, 2 * bn, 8248, "uniform", config=config, dtype=orc.FP16)
+    # what the kernel cannot run (a K of other than whole chunks, operands or a C off their boundaries) runs all the same
+    for M, N, K, offA, offC in [(bm, bn, 129, 0, 0), (bm, bn, 72, 0, 0), (bm + 3, bn, 256, 4, 0), (bm, bn + 1, 264, 0, 2)]:
+        C, ref, guard = _run_offset(mi, orc, config, M, N, K, offA, 0, offC)
+        assert (C == ref).all() and (guard == 0xEEEE).all(), (M, N, K, offA, offC)
+
+
+@pytest.mark.parametrize("M,N,K", [(300, 260, 648), (1000, 700, 2568)])
+def test_deep_ring_keeps_infinities_and_nan_in_their_rows(mi, orc, M, N, K):
+    """A row's first and last chunks share their lines with its neighbours' rows: what stands there reaches no other
+    row or column of C."""
+    from h100_gemm_amd import kernel_configs as kc
+    assert kc.CONFIGS[mi.select_config(M, N, K)].get("DEEP")
+    A, B = make_inputs(orc, M, N, K, "int")
+    A[5, K - 1], A[6, 0], A[M - 1, K - 1], B[7, K - 1], B[9, 0] = 0x7FC0, 0x7F80, 0x7F80, 0x7F80, 0x7FC0
+    C = orc.to_f32(Dev(mi, A, B, M, N).run(K))
+    finite = np.isfinite(C)
+    assert np.isnan(C[5]).all() and not finite[[6, M - 1]].any() and not finite[:, [7, 9]].any()
+    finite[[5, 6, M - 1]] = True
+    finite[:, [7, 9]] = True
+    assert finite.all()
+
+
 def test_wave_split_k_dispatch_and_determinism(mi, orc):
     from h100_gemm_amd import kernel_configs as kc
     # the automatic choice for few-tile shapes; the same answers as the tiled kernels where
