@@ -642,6 +642,12 @@ size_t launch_workgroups(const mi::KernelEntry& e, int M, int N, int splits) {
     return (size_t)((M + e.BM - 1) / e.BM) * tiles_n * (size_t)splits;
 }
 
+// ... for a call that names the config, with operands and C on 16-byte boundaries or not (C on 8 bytes: a K in pieces)
+size_t config_workgroups(int config, int M, int N, int K, bool ptr_aligned) {
+    const Choice c = compute_choice(config, M, N, K, ptr_aligned && N % 4 == 0 && K % 64 == 0, N % 4 == 0, ptr_aligned, true);
+    return launch_workgroups(mi::kKernels[c.config], M, N, c.splits);
+}
+
 // One GEMM launch (more with split-K and with a copy of the operands): argument checks, kernel choice, aligned / predicated twin.
 // `may_cut`: the automatic choice may run the shape as two GEMMs, the first rows and the rest
 // (rows_to_split_off in the kernel table); the parts themselves are not cut again.
@@ -883,20 +889,8 @@ int mi_gemm_config_grid(int config, int M, int N, int K) {
         const int tiles_n = (N + e.BN - 1) / e.BN;
         return tiles_n * choose_splits(tiles_n, K, compute_units());
     }
-    const int tiles = ((M + e.BM - 1) / e.BM) * ((N + e.BN - 1) / e.BN);
-    if (e.deep[0][0] && K <= e.deep_max_k && mi::deep_runs(K, true)) {
-        int kps = K;
-        return tiles * choose_deep_splits(e, M, N, K, N % 4 == 0, compute_units(), &kps);
-    }
-    if (e.kind == mi::KIND_WAVEK) {    // split-K pieces, assuming an aligned C and no trace buffer
-        int kps = K;
-        return tiles * choose_small_tile_splits(e, M, N, K, N % 4 == 0, compute_units(), &kps);
-    }
-    if (e.kind == mi::KIND_MFMA16) {   // split-K pieces, assuming an aligned C and no trace buffer
-        int kps = K;
-        return tiles * choose_tile_splits(e, M, N, K, N % 4 == 0, true, compute_units(), &kps);
-    }
-    return tiles;
+    // (operands and C on 16-byte boundaries)
+    return (int)config_workgroups(config, M, N, K, true);
 }
 
 int mi_gemm_select_config(int dtype, int M, int N, int K) {
@@ -920,23 +914,25 @@ int mi_gemm_row_cut(int dtype, int M, int N, int K) {
 int mi_gemm_tuned_entries(void) { return (int)tuned_entries().size(); }
 
 size_t mi_gemm_trace_words(int M, int N, int K) {
-    // enough for whichever kernel configuration ends up running the shape -- or its two
-    // parts, one after the other, where the automatic choice cuts the shape's rows
+    // enough for whichever kernel configuration ends up running the shape, with the boundaries of the
+    // operands and C as they may be (a config's call on 4- or 8-byte boundaries can be another kernel's, in
+    // more pieces) -- or its two parts, one after the other, where the automatic choice cuts the shape's rows
     auto largest = [&](int rows) {
         size_t grid = 0;
-        for (int c = 0; c < mi::kNumKernels; ++c) {
-            const size_t g = (size_t)mi_gemm_config_grid(c, rows, N, K);
-            if (g > grid) grid = g;
-        }
+        for (int c = 0; c < mi::kNumKernels; ++c)
+            for (int aligned = 0; aligned < 2; ++aligned) {
+                const size_t g = config_workgroups(c, rows, N, K, aligned != 0);
+                if (g > grid) grid = g;
+            }
         return grid;
     };
+    if (!shape_in_range(M, N, K)) return 1;
     size_t grid = largest(M);
-    if (shape_in_range(M, N, K))
-        for (int flags = 0; flags < 16; ++flags) {
-            const int m1 = rows_to_cut(M, N, K, (flags & 1) != 0 && N % 4 == 0 && K % 64 == 0, (flags & 2) != 0 && N % 4 == 0,
-                                       (flags & 4) != 0, (flags & 8) != 0);
-            if (m1 > 0 && largest(m1) + largest(M - m1) > grid) grid = largest(m1) + largest(M - m1);
-        }
+    for (int flags = 0; flags < 16; ++flags) {
+        const int m1 = rows_to_cut(M, N, K, (flags & 1) != 0 && N % 4 == 0 && K % 64 == 0, (flags & 2) != 0 && N % 4 == 0,
+                                   (flags & 4) != 0, (flags & 8) != 0);
+        if (m1 > 0 && largest(m1) + largest(M - m1) > grid) grid = largest(m1) + largest(M - m1);
+    }
     return grid * 6 + 1;
 }
 

@@ -2,14 +2,17 @@
 // libmi_gemm.so makes (its symbols come before libamdhip64's), so "launching" a kernel runs a few lines
 // here.  They follow whose operands a workspace holds: a copy or a GEMM that writes one marks it, the
 // GEMM or reduction that reads it passes the mark on to C.  Addresses are made up and never
-// dereferenced; the top byte names the call they belong to.
+// dereferenced; the top byte names the call they belong to.  Launches with a trace buffer say how many
+// of its records they write.
 //
 //   launch_order <scenario>         exit code 0, or 1 with the fault on stderr
+#include <math.h>
 #include <stdint.h>
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
 
+#include <algorithm>
 #include <atomic>
 #include <chrono>
 #include <condition_variable>
@@ -41,6 +44,8 @@ std::map<uint64_t, uint64_t> result;               // C -> call whose product it
 std::map<std::thread::id, std::set<uint64_t>> used;   // workspaces each thread's launches named
 std::vector<uint64_t> copies;                      // where operands were copied to
 std::vector<std::string> faults;
+struct Traced { uint64_t buffer; size_t records; };
+std::vector<Traced> traced;                        // launches with a trace buffer: a record per workgroup
 uint64_t next_address = kWorkspace;
 int allocation_calls = 0, fail_above_mib = 0;      // hipMalloc of more than that fails (0: never)
 bool capturing = false;
@@ -67,7 +72,7 @@ uint64_t source_of(uint64_t p) {
     return b ? owner[b] : 0;
 }
 
-int launch(const void* stub, void** args) {
+int launch(const void* stub, Dim3 grid, void** args) {
     std::string name;
     {
         std::lock_guard<std::mutex> lock(m);
@@ -89,7 +94,8 @@ int launch(const void* stub, void** args) {
             result[c] = owner[use(ws)];
         } else {                                                             // {A, B, C, ...}
             const bool decode = name.find("DecodeArgs") != std::string::npos;    // (else GemmArgs: the workspace further on)
-            memcpy(w, args[0], decode ? 32 : 80);
+            memcpy(w, args[0], 80);
+            if (const uint64_t db = decode ? w[9] : w[8]) traced.push_back({db, (size_t)grid.x * grid.y * grid.z});
             const uint64_t ws = decode ? w[3] : w[9], src = source_of(w[0]);
             if (src != source_of(w[1])) fault("A and B of different calls are multiplied");
             for (int i = 0; i < 2; ++i)
@@ -112,7 +118,7 @@ void __hipRegisterFunction(void**, const void* stub, char*, const char* name, un
     std::lock_guard<std::mutex> lock(m);
     kernels()[stub] = name;
 }
-int hipLaunchKernel(const void* stub, Dim3, Dim3, void** args, size_t, void*) { return launch(stub, args); }
+int hipLaunchKernel(const void* stub, Dim3 grid, Dim3, void** args, size_t, void*) { return launch(stub, grid, args); }
 int hipGetDevice(int* d) { *d = 0; return 0; }
 int hipDeviceGetAttribute(int* v, int, int) { *v = 256; return 0; }
 int hipGetSymbolAddress(void** p, const void*) { *p = (void*)kStatic; return 0; }
@@ -307,6 +313,44 @@ void copy_memory() {
     expect(copies.size() == 1, "no copy once there is memory again");
 }
 
+// A trace buffer of mi_gemm_trace_words has room for every call of the shape: each configuration and the
+// automatic choice, operands and C on every boundary that changes which kernel runs, in how many pieces.
+void trace_room() {
+    std::vector<Shape> shapes = {{824, 68, 27976}, {825, 72, 19456}, {160, 1280, 11832}, {232, 432, 10952}, {23, 7208, 13488},
+                                 {11, 7296, 13376}, {1000, 780, 64}, {1000, 780, 72}, {513, 257, 136}, {7000, 7000, 4096}};
+    uint64_t seed = 1;
+    auto draw = [&](double lo, double hi, int step) {
+        seed = seed * 6364136223846793005ull + 1442695040888963407ull;
+        return std::max(step, (int)(lo * pow(hi / lo, (double)(seed >> 11) / 9007199254740992.0)) / step * step);
+    };
+    for (int i = 0; i < 400; ++i) {
+        const int step = i % 4 == 0 ? 1 : i % 4 == 1 ? 64 : 8;
+        shapes.push_back({draw(1, 4096, i % 3 ? 1 : step), draw(64, 8192, step == 1 ? 1 : 4), draw(64, 30000, step)});
+    }
+    const uint64_t db = 5ull << 40;
+    for (const Shape& s : shapes) {
+        const size_t room = (mi_gemm_trace_words(s.M, s.N, s.K) - 1) / 6;
+        for (int config = -1; config < mi_gemm_num_configs(); ++config)
+            for (uint64_t a : {0, 4, 2})
+                for (uint64_t c : {0, 8, 2}) {
+                    traced.clear();
+                    mi_gemm_ex(config, 0, s.M, s.N, s.K, (const char*)A_of(1) + a, B_of(1), (char*)C_of(1) + c, (int*)db, nullptr);
+                    size_t end = 0;
+                    for (const Traced& t : traced) end = std::max(end, (size_t)(t.buffer - db) / 24 + t.records);
+                    char text[200];
+                    snprintf(text, sizeof text, "%d x %d x %d on %s, A at +%d, C at +%d: %zu records, room for %zu", s.M, s.N, s.K,
+                             config < 0 ? "auto" : mi_gemm_config_name(config), (int)a, (int)c, end, room);
+                    expect(end <= room, text);
+                    // config_grid: what a call with everything on 16-byte boundaries launches
+                    if (config >= 0 && a + c == 0 && !traced.empty()) {
+                        snprintf(text, sizeof text, "%d x %d x %d on %s: %zu workgroups, config_grid %d", s.M, s.N, s.K,
+                                 mi_gemm_config_name(config), end, mi_gemm_config_grid(config, s.M, s.N, s.K));
+                        expect(end == (size_t)mi_gemm_config_grid(config, s.M, s.N, s.K), text);
+                    }
+                }
+    }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -323,6 +367,7 @@ int main(int argc, char** argv) {
     else if (scenario == "table_busy") table_busy();
     else if (scenario == "caller_alignment") caller_alignment();
     else if (scenario == "copy_memory") copy_memory();
+    else if (scenario == "trace_room") trace_room();
     else return 2;
     for (const std::string& f : std::set<std::string>(faults.begin(), faults.end())) fprintf(stderr, "%s\n", f.c_str());
     return faults.empty() ? 0 : 1;

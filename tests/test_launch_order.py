@@ -43,3 +43,7 @@ def test_a_caller_workspace_on_any_16_byte_boundary_takes_the_copy(program):
 
 def test_memory_held_for_copies_is_bounded_and_a_failed_allocation_is_remembered(program):
     run(program, "copy_memory")
+
+
+def test_a_trace_buffer_has_room_for_every_call_of_its_shape(program):
+    run(program, "trace_room")
