@@ -40,14 +40,14 @@
 
 namespace mi {
 
-// f(integral_constant<int, 0>) ... f(integral_constant<int, N-1>), in order
-template <class F, int... Is>
+// f(integral_constant<int, FIRST>) ... f(integral_constant<int, FIRST + N - 1>), in order
+template <int FIRST, class F, int... Is>
 __device__ __forceinline__ void deep_for_each(F&& f, std::integer_sequence<int, Is...>) {
-    (f(std::integral_constant<int, Is>{}), ...);
+    (f(std::integral_constant<int, FIRST + Is>{}), ...);
 }
-template <int N, class F>
+template <int N, int FIRST = 0, class F>
 __device__ __forceinline__ void deep_for(F&& f) {
-    deep_for_each(f, std::make_integer_sequence<int, N>{});
+    deep_for_each<FIRST>(f, std::make_integer_sequence<int, N>{});
 }
 
 template <int BM_, int BN_, int NS_, int GROUP_, int DT_, bool LINES_, int OCC_ = 1>
@@ -233,18 +233,22 @@ gemm_deep_kernel(const GemmArgs p) {
             deep_for<NMMA>([&](auto idx_c) __attribute__((always_inline)) {
                 constexpr int idx = decltype(idx_c)::value;
                 mma_one(ph, idx);
-                // (the reads over the first three quarters of the MFMAs, the loads over all)
-                deep_for<NFR>([&](auto r_c) __attribute__((always_inline)) {
-                    constexpr int r = decltype(r_c)::value;
-                    if constexpr (r * NMMA * 3 / (4 * NFR) == idx) {
-                        if constexpr (last) read_one(SN{}, 0, r);
-                        else read_one(S{}, 1, r);
-                    }
-                });
-                if constexpr (last)
-                    deep_for<L>([&](auto d_c) __attribute__((always_inline)) {
-                        if constexpr (decltype(d_c)::value * NMMA / L == idx) load_one(t + NS, S{}, d_c, edge_c, std::false_type{});
+                // (read r behind MFMA r * NMMA * 3 / (4 * NFR): over the first three quarters; load d behind d * NMMA / L: over
+                // all.  Which of them this MFMA has is computed, not asked of each: every lambda is a function until it is
+                // inlined, and ten times as many took the compiler four minutes a tile)
+                constexpr int r0 = (idx * 4 * NFR + NMMA * 3 - 1) / (NMMA * 3), r1 = ((idx + 1) * 4 * NFR + NMMA * 3 - 1) / (NMMA * 3);
+                constexpr int r_end = r1 < NFR ? r1 : NFR;
+#pragma unroll
+                for (int r = r0; r < r_end; ++r) {
+                    if constexpr (last) read_one(SN{}, 0, r);
+                    else read_one(S{}, 1, r);
+                }
+                if constexpr (last) {
+                    constexpr int d0 = (idx * L + NMMA - 1) / NMMA, d1 = ((idx + 1) * L + NMMA - 1) / NMMA;
+                    deep_for<d1 - d0, d0>([&](auto d_c) __attribute__((always_inline)) {
+                        load_one(t + NS, S{}, d_c, edge_c, std::false_type{});
                     });
+                }
                 __builtin_amdgcn_sched_barrier(0);
             });
         });
