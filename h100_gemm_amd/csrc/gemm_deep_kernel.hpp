@@ -341,9 +341,11 @@ gemm_deep_kernel(const GemmArgs p) {
                     const u32x4_t v = *(const u32x4_t*)(stg + row * (TN * 2) + ((rc ^ cswz(row)) << 4));
                     const int m_loc = wm * TM + row;
                     const int n = cn0 + rc * 8;
-                    const uint32_t off = (uint32_t)(m_loc * p.ldc + n) * 2u;
+                    // (rows past M stay out by their number: row 128 and on of 2^24 columns are 2^32 bytes away, and
+                    // would come round into C below the descriptor's end)
+                    const uint32_t off = ((uint32_t)m_loc * (uint32_t)p.ldc + (uint32_t)n) * 2u;
                     if constexpr (WHOLE) {
-                        if (n < N) __builtin_amdgcn_raw_buffer_store_b128(v, rsrcC, off, 0, 2);      // non-temporal
+                        if (m_loc < rowsA && n < N) __builtin_amdgcn_raw_buffer_store_b128(v, rsrcC, off, 0, 2);      // non-temporal
                     } else if (m_loc < rowsA) {
                         if (n + 7 < N) {
                             __builtin_amdgcn_raw_buffer_store_b128(v, rsrcC, off, 0, 0);

@@ -292,6 +292,11 @@ def deep_configs():
     return [i for i, c in enumerate(kc.CONFIGS) if c.get("DEEP") and c.get("KG", 1) == 1]
 
 
+def config_bm(i):
+    from h100_gemm_amd import kernel_configs as kc
+    return kc.CONFIGS[i]["BM"]
+
+
 @pytest.mark.parametrize("config", deep_configs())
 def test_deep_ring_kernels(mi, orc, config):
     """The deep ring of whole lines: K around every count of slabs the ring, its plain trips and its last trips make
@@ -324,6 +329,35 @@ def test_deep_ring_kernels(mi, orc, config):
     for M, N, K, offA, offC in [(bm, bn, 129, 0, 0), (bm, bn, 72, 0, 0), (bm + 3, bn, 256, 4, 0), (bm, bn + 1, 264, 0, 2)]:
         C, ref, guard = _run_offset(mi, orc, config, M, N, K, offA, 0, offC)
         assert (C == ref).all() and (guard == 0xEEEE).all(), (M, N, K, offA, offC)
+
+
+@pytest.mark.parametrize("config", [i for i in deep_configs() if config_bm(i) > 128])
+def test_deep_ring_tile_rows_past_four_gigabytes_of_c(mi, orc, config):
+    """One and two rows of 16777152 columns: the tile's rows from 128 on lie 2^32 bytes behind its first and are past M."""
+    N, K, period = 16777152, 128, 4096
+    A, B = make_inputs(orc, 2, period, K, "int")
+    dB = mi.DeviceBuffer(N * K * 2)
+    L = mi._lib.load()
+    dB.copy_from(B)
+    rows = period
+    while rows < N:                                   # B's rows repeat
+        n = min(rows, N - rows)
+        assert L.mi_memcpy_d2d(dB.ptr + rows * K * 2, dB.ptr, n * K * 2) == 0
+        rows += n
+    ref = orc.reference_cpu_gemm(A, B)
+    dA = mi.DeviceBuffer.from_numpy(A)
+    for M in (1, 2):
+        dC = mi.DeviceBuffer(M * N * 2)
+        dC.fill_bytes(0xFF)
+        print(f"case M={M} N={N} K={K} config={mi.config_name(config)}", flush=True)
+        mi.gpu_gemm(mi.GemmParams(M, N, K, dA, dB, dC), config=config)
+        mi.synchronize()
+        C = dC.to_numpy((M, N), np.uint16)
+        for first in range(0, N, period):
+            n = min(period, N - first)
+            assert (C[:, first:first + n] == ref[:M, :n]).all(), (M, first)
+        dC.free()
+    dB.free()
 
 
 @pytest.mark.parametrize("M,N,K", [(300, 260, 648), (1000, 700, 2568)])
