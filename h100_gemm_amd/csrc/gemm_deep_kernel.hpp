@@ -34,6 +34,7 @@
 #include <type_traits>
 #include <utility>
 
+#include "deep_lines.hpp"
 #include "gemm_kernel.hpp"
 #include "gemm_mfma16_kernel.hpp"   // mfma_16x16x32, f32x4_t
 #include "splitk_common.hpp"        // TraceRec
@@ -99,8 +100,7 @@ gemm_deep_kernel(const GemmArgs p) {
     const int M = p.M, N = p.N;
     const int K = SPLITK ? ((p.K - k0) < p.k_per_split ? (p.K - k0) : p.k_per_split) : p.K;
     const int KT = (K + 63) / 64;                            // K steps
-    const int slabs = LINES ? KT + 1 : KT;                   // slabs the walk requests
-    const int KC = K / 8;                                    // 16-byte chunks of a row
+    const int slabs = deep_slabs(LINES, K);
 
     const int rowsA = (M - row0) < BM ? (M - row0) : BM;
     const int rowsB = (N - col0) < BN ? (N - col0) : BN;
@@ -109,17 +109,11 @@ gemm_deep_kernel(const GemmArgs p) {
     // LINES: descriptors start on the 128-byte line that holds the first row's first element
     const uint32_t misA = LINES ? (uint32_t)(uintptr_t)Ab & 127u : 0u, misB = LINES ? (uint32_t)(uintptr_t)Bb & 127u : 0u;
     // descriptors end at the last element (of this K range) of the last valid row
-    const uint32_t bytesA = misA + (uint32_t)((rowsA - 1) * p.lda + K) * 2u;
-    const uint32_t bytesB = misB + (uint32_t)((rowsB - 1) * p.ldb + K) * 2u;
+    const uint32_t bytesA = deep_bytes(misA, rowsA, p.lda, K);
+    const uint32_t bytesB = deep_bytes(misB, rowsB, p.ldb, K);
     const __amdgpu_buffer_rsrc_t rsrcA = __builtin_amdgcn_make_buffer_rsrc((void*)(Ab - misA), 0, (int)bytesA, 0x00020000);
     const __amdgpu_buffer_rsrc_t rsrcB = __builtin_amdgcn_make_buffer_rsrc((void*)(Bb - misB), 0, (int)bytesB, 0x00020000);
 
-    auto swz = [](int row) __attribute__((always_inline)) { return (row >> 1) & 7; };
-    // phase of a row: chunks between the start of its 128-byte line and its first element
-    // (rows r and r + 16 have the same: 16 rows of K % 8 == 0 elements are whole lines)
-    auto phase = [](uint32_t mis, int row, int ld) __attribute__((always_inline)) {
-        return (int)(((mis + (uint32_t)(row * ld) * 2u) >> 4) & 7u);
-    };
     // load instruction d of A (of B) of this wave fills rows (wave * LA + d) * 8 .. + 7
     const int lr = lane >> 3, lc = lane & 7;
     const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)lds;
@@ -131,20 +125,18 @@ gemm_deep_kernel(const GemmArgs p) {
         const bool a = d < LA;
         const int e = a ? d : d - LA;
         const int row = (wave * (a ? LA : LB) + e) * 8 + lr;
-        const uint32_t start = (uint32_t)(row * (a ? p.lda : p.ldb)) * 2u + (a ? misA : misB);
-        voffs[d] = (LINES ? start & ~127u : start) + (uint32_t)(lc ^ swz(row)) * 16u - (uint32_t)((e % (a ? GA : GB)) * 1024);
+        voffs[d] = deep_chunk_offset(LINES, a ? misA : misB, row, a ? rowsA : rowsB, a ? p.lda : p.ldb, lc ^ deep_swizzle(row)) -
+                   (uint32_t)((e % (a ? GA : GB)) * 1024);
     }
-    // LINES: chunks of this lane's row from its chunk of slab 0 to the row's end (> KC: the chunk lies in front of
-    // the row); chunk and phase repeat every 16 rows, so there are two of each operand, for even and odd e
+    // LINES: chunk and phase repeat every 16 rows, so there are two of each operand, for even and odd e
     int left[2][2];
 #pragma unroll
     for (int a = 0; a < 2; ++a)
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
             const int row = (wave * (a ? LA : LB) + e) * 8 + lr;
-            left[a][e] = KC + phase(a ? misA : misB, row, a ? p.lda : p.ldb) - (lc ^ swz(row));
+            left[a][e] = deep_chunks_left(a ? misA : misB, row, a ? p.lda : p.ldb, K, lc ^ deep_swizzle(row));
         }
-    constexpr uint32_t NOWHERE = 0x80000000u;                // past the end of every descriptor: no access, zeros
     auto dma = [](__amdgpu_buffer_rsrc_t rsrc, uint32_t voff, uint32_t soff, uint32_t dst) __attribute__((always_inline)) {
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                      :: "s"(dst), "v"(voff), "s"(rsrc), "s"(soff) : "memory");
@@ -154,8 +146,9 @@ gemm_deep_kernel(const GemmArgs p) {
         asm volatile("buffer_load_dwordx4 %0, %1, %2 offen offset:%3 lds"
                      :: "v"(voff), "s"(rsrc), "s"(soff), "n"(decltype(imm_c)::value) : "memory");
     };
-    // load d of slab t into stage s.  Plain: the slab lies inside every row.  Otherwise (EDGE) chunks outside
-    // their row, and slabs past the last one, come from NOWHERE (FRONT: slab 0, where some lie in front of their row).
+    // load d of slab t into stage s.  Plain: the slab lies inside every row, and the K offset is the load's scalar one.
+    // Otherwise (EDGE) it goes into the lanes' offsets, and chunks outside their row, and slabs past the last one, come
+    // from nowhere (FRONT: slab 0, where some lie in front of their row).
     auto load_one = [&](int t, auto s_c, auto d_c, auto edge_c, auto front_c) __attribute__((always_inline)) {
         constexpr int s = decltype(s_c)::value, d = decltype(d_c)::value;
         constexpr bool edge = decltype(edge_c)::value, a = d < LA;
@@ -164,13 +157,8 @@ gemm_deep_kernel(const GemmArgs p) {
         uint32_t vo = voffs[d];
         const __amdgpu_buffer_rsrc_t rs = a ? rsrcA : rsrcB;
         if constexpr (edge) {
-            // (the K offset in the lanes' offsets, which the range check compares as they are)
-            bool ok = t < slabs;
-            if constexpr (LINES) {
-                ok = left[a][e & 1] > 8 * t;
-                if constexpr (decltype(front_c)::value) ok = ok && left[a][e & 1] <= KC;
-            }
-            vo = ok ? vo + kb : NOWHERE;
+            const bool ok = LINES ? deep_chunk_inside(left[a][e & 1], t, K, decltype(front_c)::value) : t < slabs;
+            vo = ok ? vo + kb : kDeepNowhere;
             kb = 0;
         }
         const uint32_t dst = lds_base + (uint32_t)(s * STAGE + (a ? 0 : A_STAGE) + ((int)wave * (a ? LA : LB) + (e / G) * G) * 1024);
@@ -185,12 +173,12 @@ gemm_deep_kernel(const GemmArgs p) {
     bool upA[2], upB[2];
 #pragma unroll
     for (int ph = 0; ph < 2; ++ph) {
-        const int ga = (LINES ? phase(misA, l16, p.lda) : 0) + 4 * ph + q;
-        const int gb = (LINES ? phase(misB, l16, p.ldb) : 0) + 4 * ph + q;
+        const int ga = (LINES ? deep_phase(misA, l16, p.lda) : 0) + 4 * ph + q;
+        const int gb = (LINES ? deep_phase(misB, l16, p.ldb) : 0) + 4 * ph + q;
         upA[ph] = ga >= 8;
         upB[ph] = gb >= 8;
-        rdA[ph] = (wm * TM + l16) * 128 + (((ga & 7) ^ swz(l16)) << 4);
-        rdB[ph] = A_STAGE + (wn * TN + l16) * 128 + (((gb & 7) ^ swz(l16)) << 4);
+        rdA[ph] = (wm * TM + l16) * 128 + (((ga & 7) ^ deep_swizzle(l16)) << 4);
+        rdB[ph] = A_STAGE + (wn * TN + l16) * 128 + (((gb & 7) ^ deep_swizzle(l16)) << 4);
     }
 
     u32x4_t fa[2][MI], fb[2][NI];
@@ -272,7 +260,7 @@ gemm_deep_kernel(const GemmArgs p) {
     for (int r = 0; r < NFR; ++r) read_one(std::integral_constant<int, 0>{}, 0, r);
 
     // ---- NS steps a trip (the stage a compile-time index); the last trips may request chunks past the rows' ends ----
-    const int whole = LINES ? KC / 8 : KT;                   // slabs < whole lie inside every row
+    const int whole = deep_whole_slabs(LINES, K);            // slabs < whole lie inside every row
     int t = 0;
     for (; t + 2 * NS - 1 < whole; t += NS)
         deep_for<NS>([&](auto s_c) __attribute__((always_inline)) { step(t + decltype(s_c)::value, s_c, F{}); });
