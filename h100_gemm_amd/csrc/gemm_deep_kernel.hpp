@@ -329,11 +329,9 @@ gemm_deep_kernel(const GemmArgs p) {
                     const u32x4_t v = *(const u32x4_t*)(stg + row * (TN * 2) + ((rc ^ cswz(row)) << 4));
                     const int m_loc = wm * TM + row;
                     const int n = cn0 + rc * 8;
-                    // (rows past M stay out by their number: row 128 and on of 2^24 columns are 2^32 bytes away, and
-                    // would come round into C below the descriptor's end)
                     const uint32_t off = ((uint32_t)m_loc * (uint32_t)p.ldc + (uint32_t)n) * 2u;
                     if constexpr (WHOLE) {
-                        if (m_loc < rowsA && n < N) __builtin_amdgcn_raw_buffer_store_b128(v, rsrcC, off, 0, 2);      // non-temporal
+                        if (n < N) __builtin_amdgcn_raw_buffer_store_b128(v, rsrcC, off, 0, 2);      // non-temporal
                     } else if (m_loc < rowsA) {
                         if (n + 7 < N) {
                             __builtin_amdgcn_raw_buffer_store_b128(v, rsrcC, off, 0, 0);
@@ -347,7 +345,9 @@ gemm_deep_kernel(const GemmArgs p) {
                 }
             }
         };
-        const bool whole_lines = ((p.ldc & 63) | (int)((uintptr_t)p.C & 127u)) == 0;
+        // WHOLE leaves rows past M to the range check, so a tile's rows have to lie within 32-bit offsets (of 2^24 columns row
+        // 128 is 2^32 bytes away and would come round into C below the descriptor's end)
+        const bool whole_lines = ((p.ldc & 63) | (int)((uintptr_t)p.C & 127u)) == 0 && (uint64_t)p.ldc * (BM * 2) <= 0x80000000u;
         const bool scaled = p.alpha != 1.0f || p.beta != 0.0f;
         if (whole_lines) {
             if (scaled) epilogue(T{}, T{}); else epilogue(F{}, T{});
