@@ -502,6 +502,15 @@ def test_few_rows_with_a_narrow_or_a_short_b(mi):
         assert mi.config_name(mi.select_config(M, N, K)).startswith(kind), (M, N, K, mi.config_name(mi.select_config(M, N, K)))
 
 
+def test_a_row_cut_is_priced_without_the_factors_of_the_choice(mi):
+    """The lead that the 128x128 pairs get over the small tiles at a short K (100 tiles and more, 48 MB of operands at
+    most) belongs to the choice between the two: where the whole and its first rows lie on different sides of those limits, it
+    would cut a shape, or not, for nothing."""
+    for M, N, K, first in [(11704, 25928, 640, 0), (6580, 3097, 640, 6528), (2880, 5877, 640, 2816), (3868, 4352, 512, 3840),
+                           (6834, 3008, 640, 6784)]:
+        assert mi.row_cut(M, N, K) == first, (M, N, K)
+
+
 def test_which_operands_are_copied(mi):
     """Shapes on either side of the rule for the copy of ragged operands: K odd, a multiple of 8, of 16
     and of 32 (rows that straddle fewer lines), a short K; what a workspace is asked for beyond the
