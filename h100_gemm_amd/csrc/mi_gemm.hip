@@ -527,7 +527,7 @@ Choice compute_choice(int requested, int M, int N, int K, bool streamable, bool 
     // (a config that has only a deep-ring kernel runs what that cannot on 128x128 tiles)
     if (mi::kKernels[c.config].kind == mi::KIND_DEEP && !mi::deep_runs(K, ptr_aligned)) c.config = mi::kDeepTwin;
     const mi::KernelEntry& e = mi::kKernels[c.config];
-    c.deep = e.deep[0][0] && K <= e.deep_max_k && mi::deep_runs(K, ptr_aligned);
+    c.deep = mi::deep_takes(e, K, ptr_aligned);
     if (c.deep) {
         c.splits = choose_deep_splits(e, M, N, K, splittable, cus, &c.k_per_split);
     } else if (e.kind == mi::KIND_MFMA16) {

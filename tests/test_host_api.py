@@ -502,6 +502,16 @@ def test_few_rows_with_a_narrow_or_a_short_b(mi):
         assert mi.config_name(mi.select_config(M, N, K)).startswith(kind), (M, N, K, mi.config_name(mi.select_config(M, N, K)))
 
 
+def test_what_is_priced_is_what_runs(mi):
+    """Where a config's call goes to the deep ring of its tile and that kernel's time model does not hold, the choice
+    is made by figures that do: no small tiles for an output larger than both models know (8192 x 2048 x 192: 23.1 us on 96x64,
+    18.8 on 128x128), and by its own kernel's for K groups with many products and small tiles with a very long K."""
+    for M, N, K in [(6528, 6528, 128), (4096, 4096, 128), (8192, 2048, 192), (5476, 5504, 192), (9328, 8512, 128)]:
+        assert mi.config_name(mi.select_config(M, N, K)) == "m128x128_w2x2_g4_b1_o2", (M, N, K)
+    assert mi.config_name(mi.select_config(4112, 6248, 1536)) == "m256x256_w2x2_g4_b3"
+    assert mi.config_name(mi.select_config(435, 128, 18304)) == "k64x64_s4"
+
+
 def test_a_row_cut_is_priced_without_the_factors_of_the_choice(mi):
     """The lead that the 128x128 pairs get over the small tiles at a short K (100 tiles and more, 48 MB of operands at
     most) belongs to the choice between the two: where the whole and its first rows lie on different sides of those limits, it
