@@ -108,7 +108,7 @@ def check_text(name: str, text: str) -> None:
     if cfg.get("DEEP"):                         # {bf16, fp16} x {whole K, whole lines} x {plain, split-K}, traced and not
         if isa_check.check_no_scratch(name, text, r"gemm_deep_kernel") != 16:
             raise RuntimeError(f"{name}: deep-ring kernels are missing from the assembly text")
-    if cfg["KIND"] == "mfma16" and cfg.get("EFF"):
+    if cfg["KIND"] == "mfma16" and cfg.get("EFF") and cfg.get("KG", 1) == 1:     # (K groups: predicated kernels only)
         isa_check.check_no_scratch(name, text)
     isa_check.check_lds_bytes(name, text, kc.lds_bytes(cfg))
     # registers with an asm-issued load in flight are left alone (the decode kernels' ring of A fragments)

@@ -34,11 +34,20 @@ def test_m0_is_only_written_by_the_kernels_own_asm():
 
 def test_aligned_kernels_do_not_spill():
     """The accumulators live in AGPRs and the aligned variants keep everything else in VGPRs:
-    no scratch memory, for the candidates of the automatic choice."""
-    auto = [(n, t) for n, c, t in built_units(("mfma16",)) if c.get("EFF")]
+    no scratch memory, for the candidates of the automatic choice (with K groups the deep ring has the aligned calls)."""
+    auto = [(n, t) for n, c, t in built_units(("mfma16",)) if c.get("EFF") and c.get("KG", 1) == 1]
     assert len(auto) >= 5
     for name, text in auto:
         assert isa_check.check_no_scratch(name, text) >= 2
+
+
+def test_k_groups_have_predicated_kernels_only():
+    """What an aligned variant with K groups could run goes to the deep ring of the same tile: none is compiled."""
+    grouped = [(n, c, t) for n, c, t in built_units(("mfma16",)) if c.get("KG", 1) > 1]
+    assert grouped and all(c.get("DEEP") and "DEEP_MAX_K" not in c for _, c, _ in grouped)
+    for name, _, text in grouped:
+        with pytest.raises(isa_check.IsaCheckError, match="no kernel that matches"):
+            isa_check.check_no_scratch(name, text)
 
 
 def test_golden_kernels_are_checked():
