@@ -351,6 +351,18 @@ void trace_room() {
     }
 }
 
+// Every config's kernel for a call on 16-byte boundaries and for one whose A is 4 bytes off: a line each for the test to read
+void which_kernel() {
+    std::string kernel;
+    after_launch = [&](const std::string& name) { kernel = name; };
+    for (int config = 0; config < mi_gemm_num_configs(); ++config)
+        for (uint64_t a : {0, 4}) {
+            kernel = "-";
+            mi_gemm_ex(config, 0, 16, 256, 512, (const char*)A_of(1) + a, B_of(1), C_of(1), nullptr, nullptr);
+            printf("%s %d %s\n", mi_gemm_config_name(config), (int)a, kernel.c_str());
+        }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -368,6 +380,7 @@ int main(int argc, char** argv) {
     else if (scenario == "caller_alignment") caller_alignment();
     else if (scenario == "copy_memory") copy_memory();
     else if (scenario == "trace_room") trace_room();
+    else if (scenario == "which_kernel") which_kernel();
     else return 2;
     for (const std::string& f : std::set<std::string>(faults.begin(), faults.end())) fprintf(stderr, "%s\n", f.c_str());
     return faults.empty() ? 0 : 1;

@@ -144,6 +144,12 @@ def all_configs(kinds=("tile", "ring", "mfma16", "ring16"), k_groups=True):
     return [i for i, c in enumerate(kc.CONFIGS) if c["KIND"] in kinds and (k_groups or c.get("KG", 1) == 1)]
 
 
+def config_has_two_kernels(i):
+    """a deep ring for calls on 16-byte boundaries and a kernel of its own for the others"""
+    from h100_gemm_amd import kernel_configs as kc
+    return bool(kc.CONFIGS[i].get("DEEP")) and not kc.CONFIGS[i].get("DEEP_ONLY")
+
+
 def k_for(config, K):
     """K as the configuration can take it: a kernel that splits K over two groups of waves needs
     equal halves of whole 128-deep double steps, so K is rounded up to a multiple of 256 for it"""
@@ -259,7 +265,8 @@ def test_k_groups_inside_the_workgroup(mi, orc, config):
     """Eight waves as two groups that each multiply half of K of the same tile and add their
     accumulators through LDS: aligned and ragged M and N (the predicated variant), the shortest
     K (one double step per group), fp16, epilogue, trace records; K that does not divide into
-    equal halves of whole double steps is refused."""
+    equal halves of whole double steps is refused.  (On 16-byte boundaries the config's deep ring runs these;
+    the offsets below and test_kernels_whose_aligned_calls_go_to_the_deep_ring reach the K groups.)"""
     for M, N, K in [(512, 512, 256), (1536, 1536, 1536), (257, 515, 768), (1, 1, 256), (129, 127, 1280), (2048, 2048, 2048)]:
         check(mi, orc, M, N, K, "int", config=config, exact=True)
     check(mi, orc, 1024, 768, 2048, "uniform", config=config)
@@ -285,6 +292,39 @@ def test_k_groups_inside_the_workgroup(mi, orc, config):
         C, ref, guard = _run_offset(mi, orc, config, M, N, K, offA, offB, offC)
         assert (C == ref).all(), f"{int((C != ref).sum())} elements differ"
         assert (guard == 0xEEEE).all(), "bytes outside C were written"
+
+
+@pytest.mark.parametrize("config", [i for i in all_configs(("wavek", "mfma16")) if config_has_two_kernels(i)])
+def test_kernels_whose_aligned_calls_go_to_the_deep_ring(mi, orc, config):
+    """A, B or C off its 16-byte boundary: the K groups, shared rings and the wave split that share a config with a deep ring
+    run such calls, with the K it would take (whole double steps of both K groups here)"""
+    from h100_gemm_amd import kernel_configs as kc
+    bm, bn = kc.CONFIGS[config]["BM"], kc.CONFIGS[config]["BN"]
+    offsets = [(4, 0, 0), (0, 8, 0), (0, 0, 8), (12, 4, 2)]
+    for it, (M, N, K) in enumerate([(bm, bn, 256), (bm + 1, bn + 4, 512), (2 * bm - 1, 3 * bn - 4, 1280), (300, 260, 1024),
+                                    (512, 512, 768), (1, 1, 256), (777, 1000, 2048), (128, 384, 13312)]):
+        offs = offsets[it % 4]
+        print(f"case M={M} N={N} K={K} offsets {offs} config={config}", flush=True)
+        C, ref, guard = _run_offset(mi, orc, config, M, N, K, *offs)
+        assert (C == ref).all(), f"{int((C != ref).sum())} elements differ"
+        assert (guard == 0xEEEE).all(), "bytes outside C were written"
+    C, ref, guard = _run_offset(mi, orc, config, 200, 132, 512, 4, 4, 0, dtype=orc.FP16)
+    assert (C == ref).all() and (guard == 0xEEEE).all()
+    for M, N, K, dtype, alpha, beta, layout in [(1024, 768, 2048, 0, 1.0, 0.0, 0), (512, 512, 1536, orc.FP16, 0.37, 1.25, 0),
+                                                (200, 132, 512, 0, 2.0, -1.0, mi.MI_C_COL_MAJOR)]:
+        print(f"case M={M} N={N} K={K} dtype={dtype} layout={layout} config={config}", flush=True)
+        A, B = make_inputs(orc, M, N, K, "uniform", dtype)
+        d = Dev(mi, np.concatenate([np.zeros(2, np.uint16), A.ravel()]), B, M, N)
+        out = []
+        for _ in range(2):
+            mi.gemm_epilogue(mi.GemmParams(M, N, K, d.dA.ptr + 4, d.dB, d.dC, alpha, beta), config=config, dtype=dtype, c_layout=layout)
+            mi.synchronize()
+            out.append(d.dC.to_numpy((N, M) if layout else (M, N), np.uint16).copy())
+        assert (out[0] == out[1]).all()                              # fixed summation order
+        C = np.ascontiguousarray(out[0].T) if layout else out[0]
+        ref = orc.reference_cpu_gemm(A, B, alpha=alpha, beta=beta, dtype=dtype)
+        rep = orc.check_tolerance(C, ref, K, orc.max_abs(A, dtype) * abs(alpha), orc.max_abs(B, dtype), dtype)
+        assert rep["violations"] == 0 and rep["compared"] == M * N, rep
 
 
 def deep_configs():
@@ -383,8 +423,8 @@ def test_wave_split_k_dispatch_and_determinism(mi, orc):
     for M, N, K in [(512, 512, 4096), (1024, 1024, 4096), (512, 512, 4100), (512, 510, 4096), (640, 384, 3328)]:
         check(mi, orc, M, N, K, "int", exact=True)
     assert kc.CONFIGS[mi.select_config(512, 512, 4096)]["KIND"] == "wavek"
-    # the shared-ring kernels through the automatic choice (also a K that is no multiple of 64:
-    # the tiled kernels give the same answers)
+    # the configs with a shared ring through the automatic choice (their deep rings run these; also a K
+    # that is no multiple of 64)
     for M, N, K in [(1440, 1440, 1472), (1344, 1344, 1344), (1536, 1472, 320), (1440, 1440, 1480)]:
         check(mi, orc, M, N, K, "int", exact=True)
     assert kc.CONFIGS[mi.select_config(1440, 1440, 1472)].get("SHARED") == 1
@@ -1298,11 +1338,11 @@ def test_db_trace_records(mi, orc):
     cfg = mi.find_config("m128x128_w2x2_g4_b1_o2")
     rec = records(1024, 1024, 1024, cfg)
     assert len(rec) == mi.config_grid(cfg, 1024, 1024, 1024) == 64 and (rec[:, 3] == 16).all()
-    # the automatic choice on the shapes of the benchmark's other kernel families: 512^3 (small
-    # tiles on a shared ring: every unit of K), 512 x 512 x 4096 (small tiles, K split over the
+    # the automatic choice on the shapes of the benchmark's other kernel families: 512^3 (32x32
+    # tiles on a deep ring: every unit of K), 512 x 512 x 4096 (small tiles, K split over the
     # waves: wave 0's units), 16 x 8192 x 8192 (single-pass decode: wave 0's slabs), 128 x 8192 x
-    # 8192 (split-K decode: a record per column tile and piece), and a mid-sized output on the
-    # shared-ring kernel
+    # 8192 (split-K decode: a record per column tile and piece), and a mid-sized output on 96x96
+    # tiles on a deep ring
     for (M, N, K), kind, units in [((512, 512, 512), "wavek", lambda c: 512 // 64),
                                    ((512, 512, 4096), "wavek", lambda c: 4096 // 64 // 4),
                                    ((16, 8192, 8192), "stream", lambda c: 8192 // 64 // 4),
@@ -1321,6 +1361,23 @@ def test_db_trace_records(mi, orc):
         assert grid > tiles and grid % tiles == 0                       # more than one piece per tile
         rec = records(M, N, K, mi.MI_CONFIG_AUTO)
         assert len(rec) == grid, (M, N, K, len(rec), grid)
+    # off 16-byte boundaries the config's own kernel runs, in other pieces: K on 16 bytes and A 4 bytes off (a shared
+    # ring in pieces), on K groups, and on small tiles
+    for M, N, K, config in [(160, 1280, 11832, mi.MI_CONFIG_AUTO), (23, 7208, 13488, mi.find_config("k96x64_s4")),
+                            (512, 512, 1024, mi.find_config("m128x128_w2x2_g4_b1_k2")), (512, 512, 512, mi.find_config("k32x32_s4"))]:
+        print(f"case trace M={M} N={N} K={K} config={config} A at +4", flush=True)
+        A, B = make_inputs(orc, M, N, K, "int")
+        d = Dev(mi, np.concatenate([np.zeros(2, np.uint16), A.ravel()]), B, M, N)
+        words = L.mi_gemm_trace_words(M, N, K)
+        dDB = mi.DeviceBuffer(words * 4 + 4096)
+        dDB.fill_bytes(0xFF)
+        mi.gpu_gemm(mi.GemmParams(M, N, K, d.dA.ptr + 4, d.dB, d.dC), config=config, DB=dDB)
+        mi.synchronize()
+        assert (d.dC.to_numpy((M, N), np.uint16) == orc.reference_cpu_gemm(A, B)).all()
+        db = dDB.to_numpy((words + 1024,), np.int32)
+        n = int(np.argmax(db == -1))
+        assert n % 6 == 0 and 0 < n < words and (db[n:] == -1).all(), (n, words)
+        assert (db[:n].reshape(-1, 6)[:, 5] == 1).all()
     # a shape that runs as two GEMMs: the first part's records, then the second part's
     M, N, K = 7000, 7000, 4096
     m1 = mi.row_cut(M, N, K)

@@ -21,6 +21,7 @@ def program(mi, tmp_path_factory):
 def run(program, scenario):
     r = subprocess.run([str(program), scenario], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stderr
+    return r.stdout
 
 
 @pytest.mark.parametrize("source", ["library", "caller", "static"])
@@ -47,3 +48,19 @@ def test_memory_held_for_copies_is_bounded_and_a_failed_allocation_is_remembered
 
 def test_a_trace_buffer_has_room_for_every_call_of_its_shape(program):
     run(program, "trace_room")
+
+
+def test_which_of_its_kernels_a_config_runs(program):
+    """A config's deep-ring kernel takes the calls on 16-byte boundaries; 4 bytes off them its own kernel runs (that of
+    DEEP_TWIN where it has none)."""
+    from h100_gemm_amd import kernel_configs as kc
+    ran = {(name, int(a)): kernel for name, a, kernel in (line.split() for line in run(program, "which_kernel").splitlines())}
+    deep = [c for c in kc.CONFIGS if c.get("DEEP")]
+    assert len(ran) == 2 * len(kc.CONFIGS) and len(deep) == 13
+    for c in kc.CONFIGS:
+        name = kc.config_name(c)
+        assert ("gemm_deep_kernel" in ran[name, 0]) == bool(c.get("DEEP")), name
+        if c.get("DEEP"):
+            own = ("gemm_mfma16_kernel" if c["KIND"] == "mfma16" else
+                   "gemm_shared_ring_kernel" if c.get("SHARED") else "gemm_wavek_kernel")
+            assert own in ran[name, 4], (name, ran[name, 4])
