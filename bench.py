@@ -48,8 +48,7 @@ WORKLOADS = {
     # outputs of few tiles (not BASELINE configurations; for the profiles of the small-tile kernel)
     "fewtile512": (512, 512, 4096, "uniform"),
     "fewtile1024": (1024, 1024, 4096, "uniform"),
-    # 144 and 256 tiles of 128x128: one workgroup per CU at most (the kernel with two K groups)
-    # 225 tiles of 96x96, one per CU at most, K too short to split over the waves (the shared-ring kernel)
+    # 225 and 256 tiles of 96x96 and 256 of 128x128: one workgroup per CU at most (deep rings)
     "mid1440": (1440, 1440, 1472, "uniform"),
     "square1536": (1536, 1536, 1536, "uniform"),
     "square2048": (2048, 2048, 2048, "uniform"),
@@ -71,7 +70,7 @@ MEASURED_TRAFFIC_KIB = {
     "unaligned": ("m256x192_w2x2_g4_b3", "ragged_copy_and_narrow_decode.md", (127821, 31011), (49662, 62708)),   # GEMM + copy of the operands: 0.44 GB against 0.113 GB algorithmic
     "mlp_up": ("m256x256_w2x2_g4_b3", "gemm_mfma16_kernel_mlp_up.md", (2753369,), (458767,)),          # 6.1 GB against 1.34 GB algorithmic
     "mlp_down": ("m256x256_w2x2_g8_b1", "gemm_mfma16_kernel_mlp_down.md", (2752957,), (131159,)),      # 5.8 GB against 1.07 GB algorithmic
-    "square512": ("k32x32_s4", "gemm_shared_ring_kernel_square512.md", (1587,), (512,)),                     # 3.7 MB against 1.5 MB algorithmic: a copy of the rows per L2
+    "square512": ("k32x32_s4", "gemm_deep_kernel_mid_sized.md", (1569,), (565,)),                            # 3.8 MB against 1.5 MB algorithmic: a copy of the rows per L2
     "fewtile512": ("k32x32_n2", "gemm_wavek_kernel_fewtile.md", (12317,), (512,)),                     # 25.8 MB against 8.9 MB algorithmic
     "fewtile1024": ("k64x64_n2", "gemm_wavek_kernel_fewtile.md", (24627,), (2048,)),                   # 52.5 MB against 18.9 MB algorithmic
     "skinny64": ("d64x128_n4", "gemm_decode_kernel_skinny128_skinny64.md", (69689, 4114), (8192, 1024)),      # main + reduce kernels

@@ -43,7 +43,7 @@ typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 // the second hands its accumulators to the first through LDS at the end.  For tiles that are
 // alone on their CU (a lone 128x128 workgroup of the two-per-CU kernel runs at ~62 % of its
 // paired rate: two waves per SIMD hide each other's LDS and load latency).  Predicated in the library: what the
-// aligned variant could run goes to the deep ring of the same tile (0.64 / 0.71 of its time on 22 shapes of up to 6e10 products,
+// aligned variant could run goes to the deep ring of the same tile (0.76 / 0.80 of its time on 36 shapes of up to 6e10 products,
 // 0.98 / 0.97 on 41 larger ones, operands from memory / in the caches).
 template <int BM_, int BN_, int WM_, int WN_, int GROUP_, int DT_, int DRAIN_ = 0, bool EDGE_ = false, int OCC_ = 1,
           int KG_ = 1>

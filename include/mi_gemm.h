@@ -173,7 +173,9 @@ int mi_gemm_num_configs(void);
  * "t128x128_w2x2_s1_g8_o2_d1_e1" (32x32x16-MFMA kernel), "r256x256_w2x2_n4_g8" (LDS-ring
  * kernel), "s16x32_n3" / "d128x128_n3" (single-pass / split-K decode kernels), "k64x64_n2" /
  * "k96x96_s4" (small tiles for outputs of few tiles: K split over the waves of a workgroup /
- * the waves sharing one ring of LDS stages); NULL if out of range. */
+ * the waves sharing one ring of LDS stages; with K % 8 == 0, K >= 128 and 16-byte aligned operands and C
+ * the latter run a deeper ring of the same tile), "p128x96_n5" (that deep ring alone; other calls run on
+ * 128x128 tiles); NULL if out of range. */
 const char* mi_gemm_config_name(int config);
 /* Index of the config with that name, or -1. */
 int mi_gemm_find_config(const char* name);
