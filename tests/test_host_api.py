@@ -512,6 +512,15 @@ def test_what_is_priced_is_what_runs(mi):
     assert mi.config_name(mi.select_config(435, 128, 18304)) == "k64x64_s4"
 
 
+def test_a_config_keeps_its_own_price_beside_its_deep_rings(mi):
+    """The deep ring of a tile is ahead of the tile's own kernel, so the price of the latter holds for the config too: with few rows
+    it is the lower one, and without it these went to tiles split over the waves (91 x 9728 x 1664: 15.2 us for 13.0, 39 x
+    1600 x 8896 12.8 for 9.6, 46 x 3072 x 6144 15.9 for 10.9)."""
+    for M, N, K, name in [(91, 9728, 1664, "k96x64_s4"), (64, 2024, 11352, "k64x64_s4"), (39, 1600, 8896, "k64x64_s4"),
+                          (46, 3072, 6144, "k64x64_s4"), (75, 3456, 6784, "k96x96_s4"), (72, 8000, 1408, "k64x64_s4")]:
+        assert mi.config_name(mi.select_config(M, N, K)) == name, (M, N, K)
+
+
 def test_a_row_cut_is_priced_without_the_factors_of_the_choice(mi):
     """The lead that the 128x128 pairs get over the small tiles at a short K (100 tiles and more, 48 MB of operands at
     most) belongs to the choice between the two: where the whole and its first rows lie on different sides of those limits, it
