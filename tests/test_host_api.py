@@ -521,6 +521,14 @@ def test_a_config_keeps_its_own_price_beside_its_deep_rings(mi):
         assert mi.config_name(mi.select_config(M, N, K)) == name, (M, N, K)
 
 
+def test_wide_tiles_pay_for_rows_of_c_off_lines(mi):
+    """Where rows of C do not start on 128-byte lines the deep ring's 256x128 and 128x256 tiles store them 3.3 us slower, a third
+    of a call with a short K: the 128x128 pairs (912 x 6800 x 256: 9.5 us, 11.8), not so with whole lines (704 x 8896 x 256: 9.1, 8.3)."""
+    for M, N, K in [(912, 6800, 256), (3800, 1816, 256), (557, 10211, 256), (3983, 2079, 256), (2328, 3919, 256)]:
+        assert mi.config_name(mi.select_config(M, N, K)) == "m128x128_w2x2_g4_b1_o2", (M, N, K)
+    assert mi.config_name(mi.select_config(704, 8896, 256)) == "p256x128_n3"
+
+
 def test_a_row_cut_is_priced_without_the_factors_of_the_choice(mi):
     """The lead that the 128x128 pairs get over the small tiles at a short K (100 tiles and more, 48 MB of operands at
     most) belongs to the choice between the two: where the whole and its first rows lie on different sides of those limits, it
