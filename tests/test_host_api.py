@@ -529,6 +529,17 @@ def test_wide_tiles_pay_for_rows_of_c_off_lines(mi):
     assert mi.config_name(mi.select_config(704, 8896, 256)) == "p256x128_n3"
 
 
+def test_a_second_deep_ring_on_a_cu_pays_for_its_empty_ring(mi):
+    """One deep ring fills a CU's LDS, so with more tiles than CUs the next workgroup's first loads hide behind nothing: larger or
+    paired tiles (4736 x 2048 x 2048: 49.4 us on 192x128, 41.0 on 192x256; 2944 x 3200 x 128 12.1 on 256x128, 8.4 on 128x128
+    pairs); one tile a CU stays (4096 x 1536 x 1024: 192 tiles of 256x128)."""
+    for M, N, K, name in [(4736, 2048, 2048, "m192x256_w2x2_g4_b1"), (4032, 2368, 3072, "m192x256_w2x2_g4_b1"),
+                          (704, 11904, 576, "m192x192_w2x2_g4_b1"), (2944, 3200, 128, "m128x128_w2x2_g4_b1_o2"),
+                          (3391, 2368, 256, "m128x128_w2x2_g4_b1_o2")]:
+        assert mi.config_name(mi.select_config(M, N, K)) == name, (M, N, K)
+    assert mi.config_name(mi.select_config(4096, 1536, 1024)).startswith("p")
+
+
 def test_a_row_cut_is_priced_without_the_factors_of_the_choice(mi):
     """The lead that the 128x128 pairs get over the small tiles at a short K (100 tiles and more, 48 MB of operands at
     most) belongs to the choice between the two: where the whole and its first rows lie on different sides of those limits, it
